@@ -1,4 +1,5 @@
-// Matrix-core prefill GEMM for packed ternary / NF4 / INT8 weights (m > 8).
+// Matrix-core prefill GEMM for packed NF4 / INT8 weights, and for ternary ones
+// in single-half mode (m > 8; exact ternary: gemm_mx.hip).
 //
 // out[m, n] = sum_g scale[n, g] * sum_{k in g} x[m, k] * level(code[n, k]),
 // the reference's group-then-scale order (kernels-simd/src/lib.rs:54,205).
@@ -33,13 +34,11 @@
 // tiles' byte order) or k = 32h + 8q + 0..7 (NF4: its 32-wide kstep).
 //
 // Tiling.  A 256-lane block (4 waves) computes a 128 (m) x 128 (n) output
-// tile (64 x 128 where 128-row tiles would need a K split; its waves lie
-// along n), split over S weight streams of 128 / S columns each.  The waves lie
-// along n: each owns all 128 rows x 32 columns (8 x 2 MFMA tiles), so every
-// weight tile is decoded by one wave of the block; exact ternary keeps 2 x 2
-// waves of 64 x 64 (4 x 4 MFMA tiles), which reuse each activation fragment
-// over four column tiles.  A wave holds a group accumulator and a running
-// total per MFMA tile.  The 74 KB of LDS lets two blocks share a CU.
+// tile (64 x 128 where 128-row tiles would need a K split), split over S weight
+// streams of 128 / S columns each.  The waves lie along n: each owns all rows x
+// 32 columns (8 or 4 x 2 MFMA tiles), so every weight tile is decoded by one
+// wave of the block.  A wave holds a group accumulator and a running total per
+// MFMA tile.  The 74 KB of LDS lets two blocks share a CU.
 //
 // Grid mapping.  Workgroups are dealt round-robin to the 8 XCDs.  Block b
 // computes tile (b % 8) * (tiles / 8) + b / 8, so each XCD's L2 holds a
@@ -60,7 +59,7 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 256;  // 4 waves: 2 (m) x 2 (n)
+constexpr int kThreads = 256;  // 4 waves along n
 constexpr int kBM = 128;       // rows per block tile
 constexpr int kBN = 128;       // columns per block tile (all streams)
 constexpr int kBK = 64;        // k per stage
@@ -74,12 +73,6 @@ __constant__ float kLevels[16] = {
     0.0795803f,   0.1609302f,   0.2461123f,   0.33791524f,
     0.44070983f,  0.562617f,    0.72295684f,  1.0f,
 };
-
-__device__ __forceinline__ float silu_mul(float gate, float up)
-{
-    const float sigmoid = 1.0f / (1.0f + expf(-gate));
-    return (gate * sigmoid) * up;
-}
 
 __device__ __forceinline__ float wave_max(float v)
 {
@@ -246,20 +239,14 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
     constexpr int P = F == Format::Nf4 ? 2 : 1;  // weight level planes
     constexpr int PA = LO ? 2 : 1;               // activation planes (hi, lo)
     // Waves along n (M = 2048 x 8192 x 2048 against 2 x 2: NF4 exact 218 ->
-    // 206 us, INT8 exact 172 -> 165, single-half 3-9 % faster; exact ternary
-    // 158 -> 159-160, so it keeps 2 x 2 at 128 rows).
-    constexpr int WN = LO && F == Format::Ternary && BM == kBM ? 2 : 4;
+    // 206 us, INT8 exact 172 -> 165, single-half 3-9 % faster).
+    constexpr int WN = 4;
     constexpr int WM = 4 / WN;
     constexpr int TI = BM / 16 / WM;             // 16-row MFMA tiles per wave
     constexpr int TJ = kBN / 16 / WN;            // 16-column MFMA tiles per wave
     constexpr int TJS = TJ / S;                  // column tiles per stream per wave
     constexpr int BNS = kBN / S;                 // block columns per stream
     constexpr int SPC = Chunk<F>::stages;
-    // Raised wave priority over each half-stage's MFMAs for exact ternary
-    // (165 -> 157-160 us); with the waves along n every other variant ran
-    // as fast or faster without it (INT8 exact 168.6 against 165.3 us, NF4
-    // single-half 150.7 against 144.1).
-    constexpr bool PRIO = LO && F == Format::Ternary;
     __shared__ _Float16 As[2][PA][BM][kRow];   // [stage][hi, lo][row][k]
     __shared__ uint2 lut[F == Format::Nf4 ? 256 : 1];
 
@@ -415,8 +402,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
             if (h == 1 && (s + 1) % SPC == 0 && s + 1 < s_end)
                 load_chunk((s + 1) / SPC, cur);
             const int koff = F == Format::Nf4 ? 32 * h + 8 * lq : 16 * lq + 8 * h;
-            if constexpr (PRIO)
-                __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int i = 0; i < TI; ++i) {
                 const int row = wm * (BM / WM) + i * 16 + li;
@@ -437,8 +422,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
                     acc[i][jt] = c;
                 }
             }
-            if constexpr (PRIO)
-                __builtin_amdgcn_s_setprio(0);
         }
         if (!FIRST) {
             // Group epilogue: total += group_sum * scale[n].
@@ -552,11 +535,17 @@ template <Format F, int S, Epilogue E, int BM>
 void launch_rows(hipStream_t stream, const GemmArgs &args, bool half, bool lo)
 {
     const unsigned grid = args.tiles * args.chunks;
-    if (half && lo)
-        gemm_mfma_kernel<F, S, E, true, true, BM><<<grid, kThreads, 0, stream>>>(args);
-    else if (lo)
-        gemm_mfma_kernel<F, S, E, false, true, BM><<<grid, kThreads, 0, stream>>>(args);
-    else if (half)
+    // Exact ternary runs in gemm_mx.hip.
+    if constexpr (F != Format::Ternary) {
+        if (lo) {
+            if (half)
+                gemm_mfma_kernel<F, S, E, true, true, BM><<<grid, kThreads, 0, stream>>>(args);
+            else
+                gemm_mfma_kernel<F, S, E, false, true, BM><<<grid, kThreads, 0, stream>>>(args);
+            return;
+        }
+    }
+    if (half)
         gemm_mfma_kernel<F, S, E, true, false, BM><<<grid, kThreads, 0, stream>>>(args);
     else
         gemm_mfma_kernel<F, S, E, false, false, BM><<<grid, kThreads, 0, stream>>>(args);
@@ -569,12 +558,9 @@ void launch_epilogue(hipStream_t stream, const GemmArgs &args, bool half, bool l
         launch_rows<F, S, E, kBM>(stream, args, half, lo);
     else
         launch_rows<F, S, E, kBM / 2>(stream, args, half, lo);
-    if (args.chunks > 1) {
-        const size_t plane = size_t(args.m) * args.n;
-        const unsigned rgrid = unsigned(std::min<size_t>((plane + 255) / 256, 65536));
-        splitk_reduce_kernel<S, E><<<rgrid, 256, 0, stream>>>(args.out[0], args.out[1],
-                                                              args.partial, plane, args.chunks);
-    }
+    if (args.chunks > 1)
+        launch_splitk_reduce(stream, E, args.out[0], args.out[1], args.partial,
+                             size_t(args.m) * args.n, args.chunks);
 }
 
 template <Format F>
@@ -638,7 +624,32 @@ uint32_t block_rows(const PackedCall &call)
 
 }  // namespace
 
+void launch_splitk_reduce(hipStream_t stream, Epilogue epilogue, float *out_a, float *out_b,
+                          const float *partial, size_t plane, uint32_t chunks)
+{
+    const unsigned grid = unsigned(std::min<size_t>((plane + 255) / 256, 65536));
+    switch (epilogue) {
+    case Epilogue::Single:
+        splitk_reduce_kernel<1, Epilogue::Single>
+            <<<grid, 256, 0, stream>>>(out_a, out_b, partial, plane, chunks);
+        return;
+    case Epilogue::Pair:
+        splitk_reduce_kernel<2, Epilogue::Pair>
+            <<<grid, 256, 0, stream>>>(out_a, out_b, partial, plane, chunks);
+        return;
+    case Epilogue::SwigluPair:
+        splitk_reduce_kernel<2, Epilogue::SwigluPair>
+            <<<grid, 256, 0, stream>>>(out_a, out_b, partial, plane, chunks);
+        return;
+    }
+}
+
 size_t gemm_mfma_scratch_bytes(const PackedCall &call)
+{
+    return gemm_mx_served(call) ? gemm_mx_scratch_bytes(call) : gemm_halves_scratch_bytes(call);
+}
+
+size_t gemm_halves_scratch_bytes(const PackedCall &call)
 {
     uint32_t tiles_n;
     const uint32_t chunks =
@@ -651,6 +662,8 @@ size_t gemm_mfma_scratch_bytes(const PackedCall &call)
 
 void launch_gemm_mfma(hipStream_t stream, const PackedCall &call, void *scratch)
 {
+    if (gemm_mx_served(call))
+        return launch_gemm_mx(stream, call, scratch);
     const uint32_t groups = call.k / 128;
     char *p = static_cast<char *>(scratch);
     _Float16 *xh = reinterpret_cast<_Float16 *>(p);

@@ -76,6 +76,13 @@ __device__ __forceinline__ void merge(Candidate &c, float ov, uint32_t oi, int o
     }
 }
 
+// (g * (1 / (1 + exp(-g)))) * u, backend-cpu/src/packed.rs:361-362.
+__device__ __forceinline__ float silu_mul(float gate, float up)
+{
+    const float sigmoid = 1.0f / (1.0f + expf(-gate));
+    return (gate * sigmoid) * up;
+}
+
 struct PackedCall {
     Format format = Format::Ternary;
     Epilogue epilogue = Epilogue::Single;
@@ -201,6 +208,18 @@ void launch_gemm_fma(hipStream_t stream, const PackedCall &call);
 // levels, f32 group epilogue).  `scratch` holds gemm_mfma_scratch_bytes.
 size_t gemm_mfma_scratch_bytes(const PackedCall &call);
 void launch_gemm_mfma(hipStream_t stream, const PackedCall &call, void *scratch);
+// The same for ternary weights with exact activations, on the block-scaled
+// FP6 x FP4 MFMA (gemm_mx.hip): whether it serves the call, its scratch and
+// its launch.  launch_gemm_mfma and gemm_mfma_scratch_bytes choose it.
+// gemm_halves_scratch_bytes is the scratch of the binary16-halves plan.
+size_t gemm_halves_scratch_bytes(const PackedCall &call);
+bool gemm_mx_served(const PackedCall &call);
+size_t gemm_mx_scratch_bytes(const PackedCall &call);
+void launch_gemm_mx(hipStream_t stream, const PackedCall &call, void *scratch);
+// Sums the K chunks' partial products ([chunk][stream][plane]) in chunk order
+// and applies the epilogue.
+void launch_splitk_reduce(hipStream_t stream, Epilogue epilogue, float *out_a, float *out_b,
+                          const float *partial, size_t plane, uint32_t chunks);
 
 // out[i] = the binary16 value bits[i] as f32 (exact).
 void launch_f16_to_f32(hipStream_t stream, float *out, const uint16_t *bits, size_t count);

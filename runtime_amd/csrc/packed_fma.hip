@@ -92,13 +92,6 @@ __device__ __forceinline__ float wave_sum(float v)
     return v;
 }
 
-__device__ __forceinline__ float silu_mul(float gate, float up)
-{
-    // (g * (1 / (1 + exp(-g)))) * u, backend-cpu/src/packed.rs:361-362.
-    float sigmoid = 1.0f / (1.0f + expf(-gate));
-    return (gate * sigmoid) * up;
-}
-
 // ---------------------------------------------------------------------------
 // Decode GEMV: one wave owns kRows weight rows and strides the whole K range
 // with 16 weights per lane per step, so the wave's code loads are contiguous

@@ -94,12 +94,6 @@ __device__ __forceinline__ float wave_max(float v)
     return v;
 }
 
-__device__ __forceinline__ float silu_mul(float gate, float up)
-{
-    float sigmoid = 1.0f / (1.0f + expf(-gate));
-    return (gate * sigmoid) * up;
-}
-
 __device__ __forceinline__ float wave_sum_f(float v)
 {
 #pragma unroll

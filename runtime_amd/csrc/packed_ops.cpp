@@ -163,10 +163,19 @@ mfh_status run_packed(mfh_ctx *ctx, PackedCall call, const mfh_buf *codes_a,
             s = prepare_tiles(ctx, codes_b, scales_b, p, &call.b);
         if (s)
             return s;
-        void *scratch = digits_scratch(ctx, gemm_mfma_scratch_bytes(call));
-        if (!scratch)
-            return allocation_failed(ctx);
         call.single_half = ctx->gemm_activations == 1;
+        void *scratch = digits_scratch(ctx, gemm_mfma_scratch_bytes(call));
+        if (!scratch) {
+            // The digit records round the rows up to 16, so a budget that
+            // holds plain halves may refuse them: such a call still runs, on
+            // the FP32 FMA kernel, which needs no scratch.
+            if (!gemm_mx_served(call) || !digits_scratch(ctx, gemm_halves_scratch_bytes(call)))
+                return allocation_failed(ctx);
+            launch_gemm_fma(stream, call);
+            return hipGetLastError() == hipSuccess
+                       ? MFH_OK
+                       : fail(ctx, MFH_BACKEND_FAILURE, "packed kernel launch failed");
+        }
         launch_gemm_mfma(stream, call, scratch);
     } else {
         launch_gemm_fma(stream, call);
