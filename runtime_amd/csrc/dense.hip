@@ -654,6 +654,7 @@ __global__ __launch_bounds__(kBlock) void gqa_kernel(float *__restrict__ out,
 }
 
 // ---- prefill attention on fp32 matrix cores ------------------------------
+// (head width 64, the models', runs in gqa_flash.hip)
 //
 // Flash-style causal GQA for many (token, query head) pairs.  A block of
 // kFlashWaves waves serves one key/value head and kFlashRows query rows:
@@ -1573,15 +1574,15 @@ uint32_t gqa_splits(const GqaShape &g)
     return uint32_t(splits);
 }
 
-// The fp32 matrix-core prefill kernel serves heads of 16..kFlashMaxDim
-// dimensions in steps of 16, groups of at most kFlashRows query heads, and
-// 16-byte aligned operands (its float4 loads and stores).
+// The matrix-core prefill kernels serve heads of 16..kFlashMaxDim dimensions
+// in steps of 16, groups of at most kFlashRows query heads, and 16-byte aligned
+// operands (their float4 loads and stores).
 bool flash_served(const GqaShape &g, const float *out, const float *query, const float *key_cache,
                   const float *value_cache)
 {
     auto aligned = [](const float *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     return g.head_dim && g.head_dim % 16 == 0 && g.head_dim <= kFlashMaxDim && g.group >= 1 &&
-           g.group <= kFlashRows && aligned(out) && aligned(query) && aligned(key_cache) &&
+           g.group <= kFlashRows && (g.head_dim != 64 || gqa_flash_split_served(g)) && aligned(out) && aligned(query) && aligned(key_cache) &&
            aligned(value_cache);
 }
 
@@ -1597,13 +1598,14 @@ void launch_flash_d(hipStream_t stream, float *out, const float *query, const fl
 }
 
 void launch_flash(hipStream_t stream, float *out, const float *query, const float *key_cache,
-                  const float *value_cache, const GqaShape &g)
+                  const float *value_cache, const GqaShape &g, float *scratch)
 {
     switch (g.head_dim) {
     case 16: return launch_flash_d<16>(stream, out, query, key_cache, value_cache, g);
     case 32: return launch_flash_d<32>(stream, out, query, key_cache, value_cache, g);
     case 48: return launch_flash_d<48>(stream, out, query, key_cache, value_cache, g);
-    case 64: return launch_flash_d<64>(stream, out, query, key_cache, value_cache, g);
+    case 64:
+        return launch_gqa_flash_split(stream, out, query, key_cache, value_cache, g, scratch);
     case 80: return launch_flash_d<80>(stream, out, query, key_cache, value_cache, g);
     case 96: return launch_flash_d<96>(stream, out, query, key_cache, value_cache, g);
     default: return launch_flash_d<112>(stream, out, query, key_cache, value_cache, g);
@@ -1617,6 +1619,11 @@ size_t gqa_scratch_bytes(const GqaShape &g)
     const uint32_t splits = gqa_splits(g);
     return splits ? size_t(g.tokens) * g.query_heads * splits * (g.head_dim + 2) * sizeof(float)
                   : 0;
+}
+
+size_t gqa_optional_scratch_bytes(const GqaShape &g)
+{
+    return !gqa_splits(g) && gqa_flash_split_served(g) ? gqa_flash_records_bytes(g) : 0;
 }
 
 void launch_gqa(hipStream_t stream, float *out, const float *query, const float *key,
@@ -1642,7 +1649,7 @@ void launch_gqa(hipStream_t stream, float *out, const float *query, const float 
         return;
     }
     if (flash_served(g, out, query, key_cache, value_cache))
-        return launch_flash(stream, out, query, key_cache, value_cache, g);
+        return launch_flash(stream, out, query, key_cache, value_cache, g, scratch);
     const size_t lds = (size_t(g.head_dim) + kKeyChunk + kBlock) * sizeof(float);
     gqa_kernel<<<unsigned(blocks), kBlock, lds, stream>>>(out, query, key_cache, value_cache, g);
 }

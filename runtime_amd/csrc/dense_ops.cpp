@@ -718,9 +718,10 @@ mfh_status mfh_causal_gqa(mfh_ctx *ctx, mfh_buf *output, const mfh_buf *query,
     g.group = query_heads / key_value_heads;
     g.scale = 1.0f / std::sqrt(float(head_dim));
     float *partials = nullptr;
-    if (const size_t bytes = gqa_scratch_bytes(g)) {
+    const size_t need = gqa_scratch_bytes(g);
+    if (const size_t bytes = need ? need : gqa_optional_scratch_bytes(g)) {
         partials = static_cast<float *>(work_scratch(ctx, bytes));
-        if (!partials)
+        if (!partials && need)
             return allocation_failed(ctx);
     }
     launch_gqa(ctx->stream, dev_f32(output), dev_f32(query), dev_f32(key), dev_f32(value),

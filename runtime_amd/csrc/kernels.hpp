@@ -310,11 +310,23 @@ void launch_qk_norm_rope(hipStream_t stream, float *query_out, float *key_out, c
 // Appends the new rows (unless `key` is null: the caller has already written
 // them at row `initial_len` of both caches), then attends.  Few (token,
 // head) pairs over long caches take a split-key path whose partials need
-// gqa_scratch_bytes(g) bytes of `scratch` (0: no scratch used).
+// gqa_scratch_bytes(g) bytes of `scratch` (0: no scratch used).  Where that is
+// 0, gqa_optional_scratch_bytes(g) bytes may be given instead (0, or a null
+// `scratch`: none).
 size_t gqa_scratch_bytes(const GqaShape &g);
+size_t gqa_optional_scratch_bytes(const GqaShape &g);
 void launch_gqa(hipStream_t stream, float *out, const float *query, const float *key,
                 const float *value, float *key_cache, float *value_cache, const GqaShape &g,
                 float *scratch);
+// Prefill attention at head width 64 (gqa_flash.hip): whether it serves the
+// shape (operands 16-byte aligned), and its launch over caches that already
+// hold the new rows.  With `records` (gqa_flash_records_bytes, 0: none used)
+// the keys of a short launch are cut into ranges; without, they are not.
+bool gqa_flash_split_served(const GqaShape &g);
+size_t gqa_flash_records_bytes(const GqaShape &g);
+void launch_gqa_flash_split(hipStream_t stream, float *out, const float *query,
+                            const float *key_cache, const float *value_cache, const GqaShape &g,
+                            float *records);
 // One decode token's qk_norm_rope + causal_gqa (no cache append for the
 // value: its row `position` must already hold the new value), as two
 // launches.  Writes the rotated key into the key cache row `position` and

@@ -1,0 +1,147 @@
+"""The 64-wide prefill attention on split binary16 operands
+(runtime_amd/csrc/gqa_flash.hip) at the edges of its tiles and key ranges, over
+the number range, and with infinities and NaN, against 64-bit softmax.
+
+Bound.  With s = sum_d |q_d k_d| / 8 of a (row, key) pair: halves drop at most
+3 * 2^-22 of each product, twelve f32 accumulations round by 2^-24 of at most s,
+and components below 2^-18 of a row's (tile's) largest carry 2^-40 of it, so a
+score is off by at most d = 2^-20 s + 2^-38 max|k| sum|q| / 8.  Probabilities
+then move by a factor within 2 d (both in the exponent and in the sum), plus
+2^-20 for exponent, halves and sums, and values by 2^-39 of the head's largest.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.test_dense_gpu import rng_f32, run_gqa, say
+
+pytestmark = pytest.mark.gpu
+D = 64
+
+
+def reference(q, k, v, start, qh, kvh):
+    """(64-bit outputs, bound) per (token, head, dimension)."""
+    tokens, total = q.shape[0], k.shape[0]
+    q = q.astype(np.float64).reshape(tokens, qh, D)
+    k = k.astype(np.float64).reshape(total, kvh, D)
+    v = v.astype(np.float64).reshape(total, kvh, D)
+    want, bound = np.empty_like(q), np.empty_like(q)
+    hidden = np.arange(total)[None, :] > start + np.arange(tokens)[:, None]
+    for h in range(qh):
+        qq, kk, vv = q[:, h], k[:, h // (qh // kvh)], v[:, h // (qh // kvh)]
+        score = np.where(hidden, -np.inf, qq @ kk.T / 8.0)
+        p = np.exp(score - score.max(axis=1, keepdims=True))
+        p /= p.sum(axis=1, keepdims=True)
+        off = (2.0 ** -20 * (np.abs(qq) @ np.abs(kk).T) +
+               2.0 ** -38 * np.abs(kk).max() * np.abs(qq).sum(axis=1, keepdims=True)) / 8.0
+        off = np.where(hidden, 0.0, off).max(axis=1, keepdims=True)
+        want[:, h] = p @ vv
+        bound[:, h] = ((2 * off + 2.0 ** -20) * (p @ np.abs(vv)) + 2.0 ** -39 * np.abs(vv).max())
+    return want.reshape(tokens, -1), bound.reshape(tokens, -1)
+
+
+def operands(seed, tokens, start, qh, kvh):
+    cap = start + tokens
+    return (rng_f32(seed, (tokens, qh * D)), rng_f32(seed + 1, (tokens, kvh * D)),
+            rng_f32(seed + 2, (tokens, kvh * D)), rng_f32(seed + 3, (cap, kvh * D)),
+            rng_f32(seed + 4, (cap, kvh * D)))
+
+
+def check(backend, q, k, v, kc, vc, start, qh, kvh):
+    out, _, _, _ = run_gqa(backend, q, k, v, kc, vc, start, qh, kvh, D)
+    want, bound = reference(q, np.concatenate([kc[:start], k]), np.concatenate([vc[:start], v]),
+                            start, qh, kvh)
+    diff = np.abs(out.astype(np.float64) - want)
+    assert np.all(diff <= bound), f"max over bound {np.max(diff / bound):.3g}"
+
+
+# (tokens, start, query heads, kv heads): 128-row blocks of 128, 64, 42 (group
+# of three), 32 and 1 tokens with ragged last ones, 64-key tiles ending one key
+# before, at and one past an edge, and key ranges (short launches over long
+# caches), the last with a single key and with rows that see none of it.
+CASES = [(129, 0, 8, 8), (513, 0, 2, 1), (350, 5, 6, 2), (63, 0, 32, 8), (64, 0, 32, 8),
+         (65, 0, 32, 8), (33, 0, 128, 1), (32, 992, 32, 8), (40, 985, 32, 8), (64, 2000, 32, 8),
+         (300, 1000, 32, 16), (90, 2047, 16, 4), (1024, 0, 4, 1)]
+
+
+@pytest.mark.parametrize("tokens,start,qh,kvh", CASES)
+def test_edges(backend, tokens, start, qh, kvh):
+    say("flash", tokens, start, qh, kvh)
+    check(backend, *operands(9000 + tokens + start, tokens, start, qh, kvh), start, qh, kvh)
+
+
+@pytest.mark.parametrize("case", ["sharp", "tiny", "huge", "channels", "growing", "zero"])
+def test_number_range(backend, case):
+    say("flash range", case)
+    tokens, start, qh, kvh = 160, 100, 16, 4
+    q, k, v, kc, vc = operands(9100, tokens, start, qh, kvh)
+    if case == "sharp":  # one key takes nearly all of a row
+        q *= np.float32(40)
+    elif case == "tiny":
+        for a in (q, k, kc, v, vc):
+            a *= np.float32(2.0 ** -60)
+    elif case == "huge":
+        for a in (k, kc, v, vc):
+            a *= np.float32(2.0 ** 60)
+        q *= np.float32(2.0 ** -58)
+    elif case == "channels":  # dimensions of very different size
+        gain = np.exp2(np.linspace(-12, 12, D)).astype(np.float32)
+        for a in (v, vc):
+            a *= np.tile(gain, kvh)
+    elif case == "growing":  # the value scale grows from tile to tile
+        steps = np.exp2(np.arange(start + tokens) // 16).astype(np.float32)
+        vc[:start] *= steps[:start, None]
+        v *= steps[start:, None]
+    else:
+        for a in (q, k, kc, v, vc):
+            a[:] = 0
+    check(backend, q, k, v, kc, vc, start, qh, kvh)
+
+
+def test_minus_infinity_score_drops_its_key(backend):
+    """Keys at -inf under positive queries score -inf: probability zero."""
+    say("flash -inf key")
+    tokens, qh, kvh = 150, 16, 8
+    q, k, v, kc, vc = operands(9200, tokens, 0, qh, kvh)
+    q = np.abs(q) + np.float32(0.01)
+    k[70] = -np.inf
+    out, _, _, _ = run_gqa(backend, q, k, v, kc, vc, 0, qh, kvh, D)
+    keep = np.arange(tokens) != 70
+    for row in (69, 70, 71, 149):
+        seen = keep[:row + 1]
+        want, bound = reference(q[row:row + 1], k[:row + 1][seen], v[:row + 1][seen],
+                                int(seen.sum()) - 1, qh, kvh)
+        assert np.all(np.abs(out[row] - want[0]) <= bound[0])
+
+
+@pytest.mark.parametrize("what", ["key", "value", "query", "query-inf"])
+def test_non_finite_operands(backend, what):
+    say("flash non-finite", what)
+    tokens, qh, kvh = 200, 16, 8
+    q, k, v, kc, vc = operands(9300, tokens, 0, qh, kvh)
+    clean, _, _, _ = run_gqa(backend, q, k, v, kc, vc, 0, qh, kvh, D)
+    if what == "key":
+        k[130, 5] = np.nan
+    elif what == "value":
+        v[130, 5] = np.inf
+    elif what == "query":
+        q[130, 5] = np.nan
+    else:
+        q[130, 5] = np.inf
+    out, _, _, _ = run_gqa(backend, q, k, v, kc, vc, 0, qh, kvh, D)
+    out, clean = out.reshape(tokens, qh, D), clean.reshape(tokens, qh, D)
+    if what == "key":  # both query heads of key/value head 0, every row that sees it
+        assert np.isnan(out[130:, :2]).all()
+        np.testing.assert_allclose(out[:128], clean[:128], rtol=1e-4, atol=1e-5)
+        np.testing.assert_allclose(out[:, 2:], clean[:, 2:], rtol=1e-4, atol=1e-5)
+    elif what == "value":
+        assert np.isposinf(out[130:, :2, 5]).all()
+        others = [d for d in range(D) if d != 5]
+        np.testing.assert_allclose(out[:, :2][:, :, others], clean[:, :2][:, :, others], rtol=1e-4,
+                                   atol=1e-5)
+        np.testing.assert_allclose(out[:, 2:], clean[:, 2:], rtol=1e-4, atol=1e-5)
+    else:
+        assert not np.isfinite(out[130, 0]).any()
+        out[130, 0] = clean[130, 0]
+        np.testing.assert_allclose(out, clean, rtol=1e-4, atol=1e-5)
