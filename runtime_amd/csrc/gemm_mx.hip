@@ -266,7 +266,7 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
         f.start = *reinterpret_cast<const v4f *>(rec + kSumsAt + 16 * lq);
         f.exps = rec[kExpsAt + lane];
 #pragma unroll
-        for (int d = kDigits - 1; d >= 0; --d) {
+        for (int d = 0; d < kDigits; ++d) {
             f.lo[d] = *reinterpret_cast<const v4u *>(rec + d * kDigitBytes + 16 * lane);
             f.hi[d] = *reinterpret_cast<const __attribute__((address_space(3))) v2u *>(
                 hi_at[d] + i * kRecord);
@@ -332,13 +332,13 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
                 read_frag(buf, i + 1, f[(i + 1) & 1]);
             const Frag &a = f[i & 1];
 #pragma unroll
-            for (int d = kDigits - 1; d >= 0; --d) {
+            for (int d = 0; d < kDigits; ++d) {
                 const v8i ad = {int(a.lo[d][0]), int(a.lo[d][1]), int(a.lo[d][2]), int(a.lo[d][3]),
                                 int(a.hi[d][0]), int(a.hi[d][1]), 0, 0};
 #pragma unroll
                 for (int jt = 0; jt < TJ; ++jt)
                     acc[i & 1][jt] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                        ad, b[jt], d == kDigits - 1 ? a.start : acc[i & 1][jt], 2, 4, 0, a.exps, 0,
+                        ad, b[jt], d == 0 ? a.start : acc[i & 1][jt], 2, 4, 0, a.exps, 0,
                         128 - kDigitBits * d);
             }
             if (i > 0)
