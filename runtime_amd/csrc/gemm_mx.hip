@@ -42,6 +42,7 @@
 // computes tile (b % 8) * (tiles / 8) + b / 8, so each XCD's L2 holds a
 // contiguous run of tiles: neighbouring n-tiles of the same m rows.
 #include <algorithm>
+#include <type_traits>
 
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
                             lds0 + buf * (TI * kRecord) + (r * kThreads + wave * 64) * 16);
     };
 
-    // Wave-uniform tile addresses, in scalar registers.
+    // Wave-uniform tile addresses.
     const char *wptr[TJ], *sptr[TJ];
 #pragma unroll
     for (int jt = 0; jt < TJ; ++jt) {
@@ -224,25 +225,27 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
         sptr[jt] = static_cast<const char *>(g.scales[st]) +
                    live * g.groups_pad * 16 * (HALF ? 2 : 4);
     }
+    // A uniform address plus a 32-bit lane offset, both opaque: otherwise the
+    // offsets are widened outside the loop and every load adds 64 bits per lane.
+    typedef const __attribute__((address_space(1))) char *Global;
+    auto at = [](const char *base, size_t offset, uint32_t lane_offset) {
+        Global p = Global(base + offset);
+        asm volatile("" : "+s"(p), "+v"(lane_offset));
+        return p + lane_offset;
+    };
+    typedef typename std::conditional<HALF, unsigned short, float>::type Scale;
     v4u raw[TJ];
-    float gsc_next[TJ], gsc[TJ];
-    unsigned short gsc_half[TJ];
     auto load_weights = [&](uint32_t grp) {
 #pragma unroll
         for (int jt = 0; jt < TJ; ++jt)
-            raw[jt] = *reinterpret_cast<const v4u *>(wptr[jt] + size_t(grp / 2) * 1024 +
-                                                     lane * 16);
+            raw[jt] = *reinterpret_cast<const __attribute__((address_space(1))) v4u *>(
+                at(wptr[jt], size_t(grp / 2) * 1024, lane * 16));
     };
-    auto load_scales = [&](uint32_t grp) {
+    auto load_scales = [&](uint32_t grp, Scale (&dst)[TJ]) {
 #pragma unroll
-        for (int jt = 0; jt < TJ; ++jt) {
-            if constexpr (HALF)
-                gsc_half[jt] = *reinterpret_cast<const unsigned short *>(
-                    sptr[jt] + size_t(grp) * 32 + li * 2);
-            else
-                gsc_next[jt] =
-                    *reinterpret_cast<const float *>(sptr[jt] + size_t(grp) * 64 + li * 4);
-        }
+        for (int jt = 0; jt < TJ; ++jt)
+            dst[jt] = *reinterpret_cast<const __attribute__((address_space(1))) Scale *>(
+                at(sptr[jt], size_t(grp) * 16 * sizeof(Scale), li * sizeof(Scale)));
     };
 
     v4f total[TI][TJ];
@@ -273,44 +276,49 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
         }
     };
 
-    fetch(g_begin, 0);
+    fetch(g_begin, g_begin & 1);
     load_weights(g_begin);
-    load_scales(g_begin);
-    if (g_begin & 1) {  // a run that starts in the middle of a tile load
-#pragma unroll
-        for (int jt = 0; jt < TJ; ++jt)
-            raw[jt] = v4u{raw[jt][2], raw[jt][3], 0, 0};
-    }
+    Scale scale[2][TJ];
+    load_scales(g_begin, scale[0]);
+    load_scales(g_begin, scale[1]);
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     __syncthreads();
 
-    for (uint32_t grp = g_begin; grp < g_end; ++grp) {
-        const uint32_t buf = (grp - g_begin) & 1;
-        const bool more = grp + 1 < g_end;
-        // The group's weight operands and scales, then the next group's loads
-        // into the registers they leave.
+    // One group; its parity picks the half of the weight load, the LDS buffer
+    // and the scale registers, so the main loop takes two groups per iteration
+    // and moves nothing between registers.
+    auto step = [&](uint32_t grp, auto parity) {
+        constexpr int odd = decltype(parity)::value;
+        // The group's weight operands, then the next group's loads, in flight
+        // behind this one's products (the last group loads its own again).
         v8i b[TJ];
 #pragma unroll
         for (int jt = 0; jt < TJ; ++jt) {
             b[jt] = v8i{};
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const unsigned w = raw[jt][t] ^ 0x80808080u;          // canonical codes
-                b[jt][2 * t] = int(w & 0x33333333u);                  // fields 0, 2
-                b[jt][2 * t + 1] = int((w >> 2) & 0x33333333u);       // fields 1, 3
-                raw[jt][t] = raw[jt][2 + t];
+                const unsigned w = raw[jt][2 * odd + t] ^ 0x80808080u;  // canonical codes
+                b[jt][2 * t] = int(w & 0x33333333u);                    // fields 0, 2
+                b[jt][2 * t + 1] = int((w >> 2) & 0x33333333u);         // fields 1, 3
             }
-            gsc[jt] = HALF ? __half2float(__ushort_as_half(gsc_half[jt])) : gsc_next[jt];
         }
-        if (more) {
-            fetch(grp + 1, buf ^ 1);
-            load_scales(grp + 1);
-            if (grp & 1)
-                load_weights(grp + 1);
+        const uint32_t next = grp + 1 < g_end ? grp + 1 : grp;
+        if (grp + 1 < g_end)
+            fetch(grp + 1, odd ^ 1);
+        load_scales(next, scale[odd ^ 1]);
+        if (odd)
+            load_weights(next);
+        float gsc[TJ];
+#pragma unroll
+        for (int jt = 0; jt < TJ; ++jt) {
+            if constexpr (HALF)
+                gsc[jt] = __half2float(__ushort_as_half(scale[odd][jt]));
+            else
+                gsc[jt] = scale[odd][jt];
         }
 #pragma unroll
         for (int d = 0; d < kDigits; ++d) {
-            hi_at[d] = lds0 + buf * (TI * kRecord) + d * kDigitBytes + 1024 + 8 * lane;
+            hi_at[d] = lds0 + odd * (TI * kRecord) + d * kDigitBytes + 1024 + 8 * lane;
             asm volatile("" : "+v"(hi_at[d]));
         }
         Frag f[2];
@@ -322,14 +330,14 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
                 for (int r = 0; r < 4; ++r)
                     total[i][jt][r] = fmaf(acc[i & 1][jt][r], gsc[jt], total[i][jt][r]);
         };
-        read_frag(buf, 0, f[0]);
+        read_frag(odd, 0, f[0]);
         // Row tile i's products run while tile i + 1's operands are read and
         // tile i - 1's group sums are added.
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
             __builtin_amdgcn_sched_barrier(0);
             if (i + 1 < TI)
-                read_frag(buf, i + 1, f[(i + 1) & 1]);
+                read_frag(odd, i + 1, f[(i + 1) & 1]);
             const Frag &a = f[i & 1];
 #pragma unroll
             for (int d = 0; d < kDigits; ++d) {
@@ -356,7 +364,16 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
         add_group(TI - 1);
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the next stage is in LDS
         __syncthreads();
+    };
+    uint32_t grp = g_begin;
+    if (grp & 1)
+        step(grp++, std::integral_constant<int, 1>{});
+    for (; grp + 1 < g_end; grp += 2) {
+        step(grp, std::integral_constant<int, 0>{});
+        step(grp + 1, std::integral_constant<int, 1>{});
     }
+    if (grp < g_end)
+        step(grp, std::integral_constant<int, 0>{});
 
 #pragma unroll
     for (int i = 0; i < TI; ++i)
