@@ -1,5 +1,5 @@
-// Matrix-core prefill GEMM for packed NF4 / INT8 weights, and for ternary ones
-// in single-half mode (m > 8; exact ternary: gemm_mx.hip).
+// Matrix-core prefill GEMM for packed NF4 weights, and for ternary and INT8 ones
+// in single-half mode (m > 8; exact ternary: gemm_mx.hip, INT8: gemm_i8.hip).
 //
 // out[m, n] = sum_g scale[n, g] * sum_{k in g} x[m, k] * level(code[n, k]),
 // the reference's group-then-scale order (kernels-simd/src/lib.rs:54,205).
@@ -239,7 +239,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
     constexpr int P = F == Format::Nf4 ? 2 : 1;  // weight level planes
     constexpr int PA = LO ? 2 : 1;               // activation planes (hi, lo)
     // Waves along n (M = 2048 x 8192 x 2048 against 2 x 2: NF4 exact 218 ->
-    // 206 us, INT8 exact 172 -> 165, single-half 3-9 % faster).
+    // 206 us, single-half 3-9 % faster).
     constexpr int WN = 4;
     constexpr int WM = 4 / WN;
     constexpr int TI = BM / 16 / WM;             // 16-row MFMA tiles per wave
@@ -535,8 +535,8 @@ template <Format F, int S, Epilogue E, int BM>
 void launch_rows(hipStream_t stream, const GemmArgs &args, bool half, bool lo)
 {
     const unsigned grid = args.tiles * args.chunks;
-    // Exact ternary runs in gemm_mx.hip.
-    if constexpr (F != Format::Ternary) {
+    // Exact ternary and INT8 run in gemm_mx.hip and gemm_i8.hip.
+    if constexpr (F == Format::Nf4) {
         if (lo) {
             if (half)
                 gemm_mfma_kernel<F, S, E, true, true, BM><<<grid, kThreads, 0, stream>>>(args);
@@ -646,7 +646,9 @@ void launch_splitk_reduce(hipStream_t stream, Epilogue epilogue, float *out_a, f
 
 size_t gemm_mfma_scratch_bytes(const PackedCall &call)
 {
-    return gemm_mx_served(call) ? gemm_mx_scratch_bytes(call) : gemm_halves_scratch_bytes(call);
+    return gemm_mx_served(call)   ? gemm_mx_scratch_bytes(call)
+           : gemm_i8_served(call) ? gemm_i8_scratch_bytes(call)
+                                  : gemm_halves_scratch_bytes(call);
 }
 
 size_t gemm_halves_scratch_bytes(const PackedCall &call)
@@ -664,6 +666,8 @@ void launch_gemm_mfma(hipStream_t stream, const PackedCall &call, void *scratch)
 {
     if (gemm_mx_served(call))
         return launch_gemm_mx(stream, call, scratch);
+    if (gemm_i8_served(call))
+        return launch_gemm_i8(stream, call, scratch);
     const uint32_t groups = call.k / 128;
     char *p = static_cast<char *>(scratch);
     _Float16 *xh = reinterpret_cast<_Float16 *>(p);

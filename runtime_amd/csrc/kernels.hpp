@@ -208,14 +208,18 @@ void launch_gemm_fma(hipStream_t stream, const PackedCall &call);
 // levels, f32 group epilogue).  `scratch` holds gemm_mfma_scratch_bytes.
 size_t gemm_mfma_scratch_bytes(const PackedCall &call);
 void launch_gemm_mfma(hipStream_t stream, const PackedCall &call, void *scratch);
-// The same for ternary weights with exact activations, on the block-scaled
-// FP6 x FP4 MFMA (gemm_mx.hip): whether it serves the call, its scratch and
-// its launch.  launch_gemm_mfma and gemm_mfma_scratch_bytes choose it.
+// The same with exact activations for ternary weights, on the block-scaled FP6
+// x FP4 MFMA (gemm_mx.hip), and for INT8 weights, on the integer MFMA
+// (gemm_i8.hip): whether each serves the call, its scratch and its launch.
+// launch_gemm_mfma and gemm_mfma_scratch_bytes choose them.
 // gemm_halves_scratch_bytes is the scratch of the binary16-halves plan.
 size_t gemm_halves_scratch_bytes(const PackedCall &call);
 bool gemm_mx_served(const PackedCall &call);
 size_t gemm_mx_scratch_bytes(const PackedCall &call);
 void launch_gemm_mx(hipStream_t stream, const PackedCall &call, void *scratch);
+bool gemm_i8_served(const PackedCall &call);
+size_t gemm_i8_scratch_bytes(const PackedCall &call);
+void launch_gemm_i8(hipStream_t stream, const PackedCall &call, void *scratch);
 // Sums the K chunks' partial products ([chunk][stream][plane]) in chunk order
 // and applies the epilogue.
 void launch_splitk_reduce(hipStream_t stream, Epilogue epilogue, float *out_a, float *out_b,

@@ -169,7 +169,8 @@ mfh_status run_packed(mfh_ctx *ctx, PackedCall call, const mfh_buf *codes_a,
             // The digit records round the rows up to 16, so a budget that
             // holds plain halves may refuse them: such a call still runs, on
             // the FP32 FMA kernel, which needs no scratch.
-            if (!gemm_mx_served(call) || !digits_scratch(ctx, gemm_halves_scratch_bytes(call)))
+            if (!(gemm_mx_served(call) || gemm_i8_served(call)) ||
+                !digits_scratch(ctx, gemm_halves_scratch_bytes(call)))
                 return allocation_failed(ctx);
             launch_gemm_fma(stream, call);
             return hipGetLastError() == hipSuccess
