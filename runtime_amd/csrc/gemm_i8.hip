@@ -343,14 +343,15 @@ struct Plan {
     uint32_t tiles_n, tiles, chunks;
 };
 
-// The largest wave tile that still gives the launch enough blocks (400 for a
-// single product, 1000 for a pair, as measured for the ternary kernel), and for a
-// launch of one-tile waves still short of blocks K runs of at least four groups.
-// us per call, before (two binary16 passes) -> now: M = 512 x 8192 x 2048 52.8 ->
-// 48.8, 2048 x 2048 x 8192 185 -> 163, 1024 x 2048 x 2048 37.9 -> 26.6, 128 x 2048
-// x 1024 15.0 -> 10.0, 16 x 8192 x 2048 16.5 -> 11.7; M = 2048 x 8192 x 2048 177 ->
-// 178, its gate/up pair with SwiGLU 334 -> 324.  Four column tiles per wave (two
-// waves per SIMD) took 344 on that pair.  Error against 64-bit sums 5.3e-7 ->
+// The largest wave tile that still gives the launch enough blocks (400; a pair
+// that asked for 1000 took smaller tiles: M = 100 x 8192 x 2048 43 us against 29.5,
+// M = 300 x 4608 x 1024 30.4 against 23.8), and for a launch of one-tile waves still
+// short of blocks K runs of at least four groups.  us per call, before (two binary16
+// passes) -> now: M = 2048 x 2048 x 8192 185 -> 163, 1024 x 2048 x 2048 37.9 ->
+// 26.6, 128 x 2048 x 1024 15.0 -> 10.0, 16 x 8192 x 2048 16.5 -> 11.7; gate/up pairs
+// with SwiGLU M = 346 x 2560 x 1024 24.4 -> 18.4, 100 x 8192 x 2048 33.6 -> 29.5.
+// Four column tiles per wave (two waves per SIMD instead of four) took 344 against
+// 324 us on the pair M = 2048 x 8192 x 2048.  Error against 64-bit sums 5.3e-7 ->
 // 2.7e-7 (2048 x 8192 x 2048).
 Plan plan_of(const PackedCall &call)
 {
@@ -362,7 +363,7 @@ Plan plan_of(const PackedCall &call)
         p.tiles = p.tiles_n * ((row_tiles + ti - 1) / ti);
         return p;
     };
-    const uint32_t enough = s == 1 ? 400 : 1000;
+    constexpr uint32_t enough = 400;
     Plan p = with(2, 2);
     if (p.tiles < enough)
         p = with(1, 2);
@@ -408,9 +409,17 @@ size_t records_bytes(const PackedCall &call)
 
 }  // namespace
 
+// The binary16-halves kernel keeps the launches that fill the device with its
+// 64-row tiles over wide outputs: M = 512 x 8192 x 2048 46.5 us there, 48.9 here, M
+// = 2048 x 8192 x 2048 177 both, against 58 and 46 at M = 2048 x 2048 x 2048 (as
+// many blocks, fewer columns) and 185 and 163 at M = 2048 x 2048 x 8192.
 bool gemm_i8_served(const PackedCall &call)
 {
-    return call.format == Format::Int8 && !call.single_half;
+    const uint32_t columns = call.epilogue == Epilogue::Single ? 128 : 64;
+    const uint64_t blocks =
+        uint64_t((call.m + 31) / 32) * ((uint64_t(call.n) + columns - 1) / columns);
+    return call.format == Format::Int8 && !call.single_half &&
+           (call.n < 4096 || blocks < 1024);
 }
 
 size_t gemm_i8_scratch_bytes(const PackedCall &call)

@@ -1,5 +1,6 @@
-// Matrix-core prefill GEMM for packed NF4 weights, and for ternary and INT8 ones
-// in single-half mode (m > 8; exact ternary: gemm_mx.hip, INT8: gemm_i8.hip).
+// Matrix-core prefill GEMM for packed NF4 weights, for INT8 ones where gemm_i8.hip
+// does not serve the call, and for ternary ones in single-half mode (m > 8; exact
+// ternary: gemm_mx.hip).
 //
 // out[m, n] = sum_g scale[n, g] * sum_{k in g} x[m, k] * level(code[n, k]),
 // the reference's group-then-scale order (kernels-simd/src/lib.rs:54,205).
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
     constexpr int P = F == Format::Nf4 ? 2 : 1;  // weight level planes
     constexpr int PA = LO ? 2 : 1;               // activation planes (hi, lo)
     // Waves along n (M = 2048 x 8192 x 2048 against 2 x 2: NF4 exact 218 ->
-    // 206 us, single-half 3-9 % faster).
+    // 206 us, INT8 exact 172 -> 165, single-half 3-9 % faster).
     constexpr int WN = 4;
     constexpr int WM = 4 / WN;
     constexpr int TI = BM / 16 / WM;             // 16-row MFMA tiles per wave
@@ -535,8 +536,8 @@ template <Format F, int S, Epilogue E, int BM>
 void launch_rows(hipStream_t stream, const GemmArgs &args, bool half, bool lo)
 {
     const unsigned grid = args.tiles * args.chunks;
-    // Exact ternary and INT8 run in gemm_mx.hip and gemm_i8.hip.
-    if constexpr (F == Format::Nf4) {
+    // Exact ternary runs in gemm_mx.hip.
+    if constexpr (F != Format::Ternary) {
         if (lo) {
             if (half)
                 gemm_mfma_kernel<F, S, E, true, true, BM><<<grid, kThreads, 0, stream>>>(args);
