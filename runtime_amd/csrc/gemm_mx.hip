@@ -24,7 +24,13 @@
 // Bound and split.  FP6 x FP4 runs at four times the binary16 rate (measured
 // 8.2 against 2.27 PFLOP/s with eight waves per CU), so five passes cost 1.25
 // binary16 passes where hi + lo halves cost two, and the weights need no
-// decode to halves.
+// decode to halves.  us per call, halves -> digits: M = 2048 x 8192 x 2048 160 ->
+// 107, 2048 x 2048 x 8192 174 -> 117, 512 x 8192 x 2048 50 -> 31, 128 x 4608 x 1024
+// 19.9 -> 10.4.  The matrix pipe is busy 46 % of the first; vector work hardly
+// overlaps these MFMAs (four FMAs beside one take its slot from 20 to 32 cycles),
+// so the inner loop keeps to 68 vector instructions per 40 MFMAs (118 before it
+// took two groups per iteration: 111 us).  Loading two groups ahead over three
+// LDS buffers needs a second register set and leaves two waves per SIMD: 117 us.
 //
 // Operands.  The weights are read from the decode GEMV's repacked tiles (16
 // rows x K per tile, one 16-byte load per lane covering 256 k) straight into
@@ -74,7 +80,8 @@ constexpr uint32_t kMaxRowTiles = 2;
 
 // One wave per (group, 16-row tile).  Lane 16q + i holds row i, k = 16q + 0..15
 // and 64 + 16q + 0..15 of the group: the 32 k of lane block q of a repacked
-// ternary tile.
+// ternary tile.  Bound by memory at size (2048 x 8192 values, 131 MB read and
+// written: 22-27 us, 4.9-6 TB/s), by its own latency at 128 x 1024 (4.6 us).
 __global__ __launch_bounds__(kThreads) void mx_split_kernel(const float *__restrict__ x,
                                                             uint32_t m, uint32_t k,
                                                             uint32_t row_tiles, uint32_t records,
