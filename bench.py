@@ -319,17 +319,22 @@ GEMM_MS = [512, 2048]
 GEMM_SHAPES = [(8192, 2048), (2048, 8192)]
 F16_MFMA_PEAK_TFLOPS = 2500.0
 FP32_PEAK_TFLOPS = 157.3
-# MFMA products issued per algorithmic product: activations as binary16
-# hi + lo, NF4 levels as hi + lo without the lo * lo term; with the opt-in
-# single-half activations (mfh_set_gemm_activations(1)) one fewer.
-MFMA_PASSES = {"ternary": 2, "int8": 2, "nf4": 3}
+# Matrix-core time per algorithmic product, in binary16 MFMAs: ternary takes
+# five FP6 x FP4 passes at four times the binary16 rate; INT8 three 8-bit digits
+# at twice it, or binary16 hi + lo activations from 4096 columns at these sizes;
+# NF4 hi + lo halves of both sides without the lo * lo term.  The opt-in
+# single-half activations (mfh_set_gemm_activations(1)) are binary16 throughout.
+def mfma_passes(fmt: str, n: int) -> float:
+    return {"ternary": 1.25, "int8": 2 if n >= 4096 else 1.5, "nf4": 3}[fmt]
+
+
 MFMA_PASSES_SINGLE = {"ternary": 1, "int8": 1, "nf4": 2}
 
 
 def prefill_gemm(backend, reps: int = 20, warm: int = 10, sustain_ms: float = 30.0,
                  cpu: bool = True) -> dict:
     """Packed GEMM at M in {512, 2048} x {8192x2048, 2048x8192} x 3 formats
-    on the matrix-core kernel (exact hi + lo activations, the default, and
+    on the matrix-core kernels (exact activations, the default, and
     the opt-in single-half activations) and on the FP32-FMA kernel (seeded
     N(0, 0.02) weights, N(0, 1) activations).  Each case runs `warm`
     back-to-back launches and times `reps` more (HIP events): `*_cold_us`.
@@ -340,7 +345,7 @@ def prefill_gemm(backend, reps: int = 20, warm: int = 10, sustain_ms: float = 30
     window reports the start of a run rather than its rate.  Reports
     algorithmic TFLOP/s (2*M*N*K) of the sustained rate, its fraction of the
     dense f16 MFMA peak, and the fraction counting the MFMA products
-    actually issued (hi/lo passes)."""
+    actually issued (mfma_passes)."""
     from runtime_amd import convert, hiptime
     from runtime_amd.backend import WEIGHT
 
@@ -380,7 +385,7 @@ def prefill_gemm(backend, reps: int = 20, warm: int = 10, sustain_ms: float = 30
                     row[label + "_us"] = round(us, 1)
                     row[label + "_TFLOPs"] = round(2 * m * n * k / (us / 1e6) / 1e12, 1)
                 row["mfma_util"] = round(row["mfma_TFLOPs"] / F16_MFMA_PEAK_TFLOPS, 4)
-                row["mfma_issued_util"] = round(row["mfma_util"] * MFMA_PASSES[fmt], 4)
+                row["mfma_issued_util"] = round(row["mfma_util"] * mfma_passes(fmt, n), 4)
                 row["mfma_single_util"] = round(row["mfma_single_TFLOPs"] / F16_MFMA_PEAK_TFLOPS, 4)
                 row["mfma_single_issued_util"] = round(
                     row["mfma_single_util"] * MFMA_PASSES_SINGLE[fmt], 4)
