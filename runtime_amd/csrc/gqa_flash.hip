@@ -543,6 +543,7 @@ constexpr uint32_t kResident = 512;
 // tiles, whose records a second launch merges: 64 tokens over 2000 keys (32 / 8
 // heads) 112 -> 24 us, 1024 over 1024 (16 / 4) 111 -> 57.  Fuller launches lose
 // by the records' traffic (2048 tokens 101 unsplit, 141 in two ranges).
+// Of a served call: at least one token, so at least one block.
 Grid grid_of(const GqaShape &g, bool records)
 {
     Grid d;
@@ -566,7 +567,7 @@ Grid grid_of(const GqaShape &g, bool records)
 
 bool gqa_flash_split_served(const GqaShape &g)
 {
-    return g.head_dim == kDim && g.group >= 1 && g.group <= kRows &&
+    return g.tokens >= 1 && g.head_dim == kDim && g.group >= 1 && g.group <= kRows &&
            g.key_value_heads <= 65536 && g.initial_len + g.tokens < (uint64_t(1) << 31);
 }
 

@@ -145,3 +145,15 @@ def test_non_finite_operands(backend, what):
         assert not np.isfinite(out[130, 0]).any()
         out[130, 0] = clean[130, 0]
         np.testing.assert_allclose(out, clean, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("group", [4, 128])
+@pytest.mark.parametrize("prefix", [0, 64, 100])
+def test_no_tokens(backend, prefix, group):
+    """A call without tokens returns, and leaves caches and length alone."""
+    say("flash no tokens", prefix, group)
+    q, k, v, kc, vc = (a[:rows] for a, rows in zip(operands(9400, 128, 0, group, 1),
+                                                   (0, 0, 0, 128, 128)))
+    out, keys, values, length = run_gqa(backend, q, k, v, kc, vc, prefix, group, 1, D)
+    assert out.shape == (0, group * D) and length == prefix
+    assert np.array_equal(keys, kc) and np.array_equal(values, vc)
