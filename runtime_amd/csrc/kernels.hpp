@@ -16,7 +16,8 @@ struct PackedStream {
     const uint16_t *scales16 = nullptr;  // binary16 copy of `scales`, or null
     const uint8_t *tiles = nullptr;      // backend-private repacked codes, or null
     const void *tiled_scales = nullptr;  // scales in tile order, or null
-    bool tiled_half = false;             // tiled_scales holds binary16 values
+    // tiled_scales holds binary16 values (the same for every stream of a call).
+    bool tiled_half = false;
 };
 
 enum class Epilogue : int {

@@ -67,18 +67,24 @@ PackedStream stream_of(const mfh_buf *codes, const mfh_buf *scales)
 // buffer, each charged to its buffer's allocation class and bounded by the
 // context's limits.  Both are stream-ordered kernels; nothing synchronizes.
 // Nothing is replaced unless both new copies could be allocated.
+//
+// The tiled scales hold binary16 values where the buffer has them and
+// `half_allowed`: a kernel reads all of its streams at one width, so a pair
+// whose other stream has only f32 scales allows none.  An f32 copy serves
+// every later call too, and stays.
 mfh_status prepare_tiles(mfh_ctx *ctx, const mfh_buf *codes_c, const mfh_buf *scales_c,
-                         const Packed &p, PackedStream *stream)
+                         const Packed &p, PackedStream *stream, bool half_allowed = true)
 {
     // Derived copies are caches on immutable inputs; the handles stay const
     // to callers.
     mfh_buf *codes = const_cast<mfh_buf *>(codes_c);
     mfh_buf *scales = const_cast<mfh_buf *>(scales_c);
     const int fmt = int(p.format);
-    const bool half = scales->f16_shadow != nullptr;
     const bool need_codes = !codes->repacked || codes->repacked_format != fmt;
-    const bool need_scales =
-        !scales->tiled_scales || scales->tiled_format != fmt || scales->tiled_half != half;
+    const bool need_scales = !scales->tiled_scales || scales->tiled_format != fmt ||
+                             (scales->tiled_half && !half_allowed);
+    const bool half =
+        need_scales ? scales->f16_shadow != nullptr && half_allowed : scales->tiled_half;
     void *tiles = nullptr, *tiled = nullptr;
     size_t tiles_cap = 0, tiled_cap = 0;
     mfh_status s = MFH_OK;
@@ -125,6 +131,22 @@ bool use_mfma_gemv(const mfh_ctx *ctx, const PackedCall &call)
     return call.m <= 8 && ctx->kernel_path != 1 && gemv_mfma_supported(call.format);
 }
 
+// The tile copies of both streams (b only for two-stream calls).
+mfh_status prepare_streams(mfh_ctx *ctx, PackedCall *call, const mfh_buf *codes_a,
+                           const mfh_buf *scales_a, const mfh_buf *codes_b,
+                           const mfh_buf *scales_b)
+{
+    const Packed p{call->n, call->k, call->format};
+    const bool half = scales_a->f16_shadow && (!codes_b || scales_b->f16_shadow);
+    mfh_status s = prepare_tiles(ctx, codes_a, scales_a, p, &call->a, half);
+    if (!s && codes_b)
+        // An f32 copy of an earlier mixed pair needs one here as well.
+        s = prepare_tiles(ctx, codes_b, scales_b, p, &call->b, half && call->a.tiled_half);
+    if (!s && codes_b && call->a.tiled_half != call->b.tiled_half)
+        s = prepare_tiles(ctx, codes_a, scales_a, p, &call->a, false);
+    return s;
+}
+
 // Enqueue the kernels of one admitted packed product.  `a`/`b` are the
 // weight operands (b only for two-stream calls).
 mfh_status run_packed(mfh_ctx *ctx, PackedCall call, const mfh_buf *codes_a,
@@ -142,11 +164,7 @@ mfh_status run_packed(mfh_ctx *ctx, PackedCall call, const mfh_buf *codes_a,
         return MFH_OK;
     }
     if (use_mfma_gemv(ctx, call)) {
-        Packed p{call.n, call.k, call.format};
-        mfh_status s = prepare_tiles(ctx, codes_a, scales_a, p, &call.a);
-        if (!s && codes_b)
-            s = prepare_tiles(ctx, codes_b, scales_b, p, &call.b);
-        if (s)
+        if (mfh_status s = prepare_streams(ctx, &call, codes_a, scales_a, codes_b, scales_b))
             return s;
         void *scratch = digits_scratch(ctx, gemv_mfma_scratch_bytes(call));
         if (!scratch)
@@ -157,11 +175,7 @@ mfh_status run_packed(mfh_ctx *ctx, PackedCall call, const mfh_buf *codes_a,
         launch_gemv_fma(stream, call);
     } else if (ctx->kernel_path != 1) {
         // The GEMM reads the same repacked tiles as the decode GEMV.
-        Packed p{call.n, call.k, call.format};
-        mfh_status s = prepare_tiles(ctx, codes_a, scales_a, p, &call.a);
-        if (!s && codes_b)
-            s = prepare_tiles(ctx, codes_b, scales_b, p, &call.b);
-        if (s)
+        if (mfh_status s = prepare_streams(ctx, &call, codes_a, scales_a, codes_b, scales_b))
             return s;
         call.single_half = ctx->gemm_activations == 1;
         void *scratch = digits_scratch(ctx, gemm_mfma_scratch_bytes(call));
@@ -376,13 +390,12 @@ mfh_status admit_packed_linear(mfh_ctx *ctx, mfh_buf *output, const mfh_buf *inp
 bool prepared_stream(const mfh_buf *codes, const mfh_buf *scales, Format format,
                      PackedStream *stream)
 {
-    const bool half = scales->f16_shadow != nullptr;
     if (!codes->repacked || codes->repacked_format != int(format) || !scales->tiled_scales ||
-        scales->tiled_format != int(format) || scales->tiled_half != half)
+        scales->tiled_format != int(format))
         return false;
     stream->tiles = static_cast<const uint8_t *>(codes->repacked);
     stream->tiled_scales = scales->tiled_scales;
-    stream->tiled_half = half;
+    stream->tiled_half = scales->tiled_half;
     return true;
 }
 

@@ -638,6 +638,42 @@ def test_pair_ffn_shape(backend, path, scheme, m, n, k):
         buf.release()
 
 
+@pytest.mark.parametrize("scheme", SCHEMES)
+@pytest.mark.parametrize("first_exact", [True, False])
+@pytest.mark.parametrize("m,n,k", [(1, 2053, 1024), (1, 4608, 2048), (2, 320, 768),
+                                   (5, 320, 1024), (8, 1000, 2048), (9, 130, 384),
+                                   (100, 320, 768), (300, 2600, 256)])
+def test_pair_of_scales_stored_at_two_widths(backend, path, scheme, first_exact, m, n, k):
+    """One stream's scales are binary16 values (which the backend keeps at
+    that width), the other's are not; afterwards each serves products of its
+    own and pairs with streams of either width."""
+    say("pair of widths", scheme, path, first_exact, m, n, k)
+    ca, sa = make_weights(n, k, scheme, 0x5EED0420)
+    cb, sb = make_weights(n, k, scheme, 0x5EED0421)
+    cc, sc = make_weights(n, k, scheme, 0x5EED0422)
+    if first_exact:
+        sb = sb * np.float32(1.0001)
+    else:
+        sa = sa * np.float32(1.0001)
+    x = convert.normal((m, k), 0xAC70420 + m)
+    weights = [(ca, sa), (cb, sb), (cc, sc)]
+    a, b, c = (upload_weights(backend, *w) for w in weights)
+    want = [oracle.packed_linear_threaded(x, *w) for w in weights]
+    xb = backend.upload_f32(x.shape, x)
+    outs = [backend.allocate_f32((m, n)) for _ in range(2)]
+    for u, v, i, j in [(a, b, 0, 1), (c, a, 2, 0), (b, c, 1, 2)]:
+        backend.packed_linear_pair(*outs, xb, *u, *v)
+        assert_close(backend.read(outs[0]), want[i])
+        assert_close(backend.read(outs[1]), want[j])
+    for w, y in zip((a, b, c), want):
+        backend.packed_linear(outs[0], xb, *w)
+        assert_close(backend.read(outs[0]), y)
+    backend.packed_swiglu_pair(outs[0], xb, *a, *b)
+    assert_close(backend.read(outs[0]), oracle.packed_swiglu_pair(x, ca, sa, cb, sb))
+    for buf in (*a, *b, *c, xb, *outs):
+        buf.release()
+
+
 # --- gather -----------------------------------------------------------------------
 
 @pytest.mark.parametrize("scheme", SCHEMES)
