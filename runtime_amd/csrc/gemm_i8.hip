@@ -12,6 +12,10 @@
 //   the group's sum is that times 256 plus the lowest digit's, in f32, and one
 //   FMA adds it times unit * scale.
 // - A group with a non-finite value gets a NaN unit, so the row's outputs are NaN.
+// - A unit times a scale stays normal for group maxima from 2^-40 on (and f32
+//   scales of 2^-60 to 2^22).  Elsewhere the range plan of digits.hpp applies: the
+//   unit is rounded up to 14 bits, its code is those and its exponent, and the
+//   second pass multiplies mantissas and adds exponents.
 //
 // Bound and split.  Integer MFMAs run at twice the binary16 rate, so three
 // digits cost 1.5 binary16 passes where hi + lo halves cost two, and the codes
@@ -28,6 +32,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include "digits.hpp"
 #include "kernels.hpp"
 
 namespace mfh {
@@ -40,6 +45,9 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kThreads = 256;
 constexpr int kDigits = 3;
 constexpr float kLargest = 8355711.0f;  // 0x7f7f7f
+constexpr int kSmall = -40;             // a group below 2^kSmall stores a unit code
+constexpr uint32_t kCodeMask = 0x3ff;   // mantissa bits a coded unit leaves out
+constexpr int kCodeBias = 200;          // of its exponent, -172..-63
 // One digit's operands of 16 rows x 128 k: two 64-wide ksteps of 16 bytes per
 // lane.
 constexpr uint32_t kDigitBytes = 2 * 64 * 16;
@@ -85,7 +93,18 @@ __global__ __launch_bounds__(kThreads) void i8_split_kernel(const float *__restr
     int e = 0;
     if (mx > 0.0f && !bad)
         mx = frexpf(mx, &e);
-    const float units = mx > 0.0f && !bad ? kLargest / mx : 0.0f;  // per 2^e
+    float units = mx > 0.0f && !bad ? kLargest / mx : 0.0f;  // per 2^e
+    const bool small = units > 0.0f && e <= kSmall;
+    uint32_t code = 0;
+    if (__builtin_expect(__any(small), 0)) {
+        // 1 / units, in [2^-24, 2^-22], rounded up to 14 bits.
+        const uint32_t up = (__float_as_uint(1.0f / units) + kCodeMask) & ~kCodeMask;
+        const int exponent = int(up >> 23) - 127 + e + kCodeBias;  // 28..137
+        if (small) {
+            units = 1.0f / __uint_as_float(up);
+            code = uint32_t(exponent) << 13 | ((up & 0x7fffffu) >> 10);
+        }
+    }
     uint8_t *out = dst + size_t(record) * kRecord + 16 * lane;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -115,7 +134,7 @@ __global__ __launch_bounds__(kThreads) void i8_split_kernel(const float *__restr
     }
     if (q == 0)
         *reinterpret_cast<float *>(dst + size_t(record) * kRecord + kUnitsAt + 4 * i) =
-            bad ? __builtin_nanf("") : units > 0.0f ? ldexpf(1.0f / units, e) : 0.0f;
+            bad || code ? nan_of(code) : units > 0.0f ? ldexpf(1.0f / units, e) : 0.0f;
 }
 
 struct I8Args {
@@ -132,20 +151,6 @@ struct I8Args {
     uint32_t tiles_n, tiles;   // output block tiles along n, and in all
     uint32_t chunks, chunk_groups;
 };
-
-// 16 bytes per lane, from base + offset (uniform base, the lane's byte offset)
-// to the LDS bytes [lds, lds + 1024) of the wave.  The caller waits (vmcnt)
-// and synchronises before the bytes are read.  Nothing else in this file uses
-// m0.
-__device__ __forceinline__ void copy_to_lds(const uint8_t *base, uint32_t offset, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "s_nop 0\n\t"
-                 "global_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds), "v"(offset), "s"(base)
-                 : "memory");
-}
 
 template <int S, Epilogue E, bool HALF, int TI, int TJ>
 __global__ __launch_bounds__(kThreads, 3) void gemm_i8_kernel(I8Args g)
@@ -243,6 +248,7 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_i8_kernel(I8Args g)
     fetch(g_begin, 0);
     load_weights(g_begin, wts[0]);
     load_scales(g_begin, scale[0]);
+    uint32_t odd_scale = 0;  // f32 scales: set by one outside the first pass's range
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     __syncthreads();
 
@@ -260,10 +266,13 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_i8_kernel(I8Args g)
         float gsc[TJ];
 #pragma unroll
         for (int jt = 0; jt < TJ; ++jt) {
-            if constexpr (HALF)
+            if constexpr (HALF) {
                 gsc[jt] = __half2float(__ushort_as_half(scale[odd][jt]));
-            else
+            } else {
                 gsc[jt] = scale[odd][jt];
+                odd_scale |= gsc[jt] != 0.0f && !(fabsf(gsc[jt]) >= 0x1p-60f &&
+                                                  fabsf(gsc[jt]) <= 0x1p22f);
+            }
         }
         Frag f[2];
         read_frag(odd, 0, f[0]);
@@ -305,6 +314,68 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_i8_kernel(I8Args g)
     }
     if (grp < g_end)
         step(grp, std::integral_constant<int, 0>{});
+
+    // NaN totals (of rows that exist: the records past the last are no rows).
+    float nan = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+        if (mt0 + i < g.row_tiles) {
+#pragma unroll
+            for (int jt = 0; jt < TJ; ++jt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    nan += total[i][jt][r];
+        }
+    if (__builtin_expect(__any(nan != nan || odd_scale), 0)) {
+        // A tile at a time, straight from memory.
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int jt = 0; jt < TJ; ++jt) {
+                if (mt0 + i >= g.row_tiles)
+                    continue;
+                v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                for (uint32_t gr = g_begin; gr < g_end; ++gr) {
+                    const uint8_t *rec = x_src + gr * x_step + i * kRecord;
+                    const char *w = wptr[jt] + size_t(gr) * 2048 + 16 * lane;
+                    const char *sp = sptr[jt] + (size_t(gr) * 16 + li) * sizeof(Scale);
+                    float gs;
+                    if constexpr (HALF)
+                        gs = __half2float(*reinterpret_cast<const __half *>(sp));
+                    else
+                        gs = *reinterpret_cast<const float *>(sp);
+                    int gs_exp = 0;
+                    const float gs_frac = frexpf(gs, &gs_exp);
+                    v4i digit[kDigits];
+#pragma unroll
+                    for (int d = 0; d < kDigits; ++d) {
+                        digit[d] = v4i{0, 0, 0, 0};
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+                            digit[d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                                *reinterpret_cast<const v4i *>(rec + d * kDigitBytes + 1024 * h +
+                                                               16 * lane),
+                                *reinterpret_cast<const v4i *>(w + 1024 * h), digit[d], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float whole = fmaf(float((digit[0][r] << 8) + digit[1][r]), 256.0f,
+                                                 float(digit[2][r]));
+                        const uint32_t unit =
+                            reinterpret_cast<const uint32_t *>(rec + kUnitsAt)[4 * lq + r];
+                        int exp = 0;
+                        float frac = frexpf(__uint_as_float(unit), &exp);
+                        if (is_code(unit)) {
+                            exp = int((unit >> 13) & 511) - kCodeBias;
+                            frac = __uint_as_float(0x3f800000u | (unit & 0x1fffu) << 10);
+                        }
+                        sum[r] += ldexpf(whole * (frac * gs_frac), exp + gs_exp);
+                    }
+                }
+                total[i][jt] = sum;
+            }
+    }
 
 #pragma unroll
     for (int i = 0; i < TI; ++i)

@@ -22,14 +22,14 @@ from tests.test_resources_gpu import MIB, total
 pytestmark = pytest.mark.gpu
 
 
-def check(got, x, codes, scales):
+def check(got, x, codes, scales, floor=0.0):
     groups = scales.shape[1]
     w = codes.view(np.int8).astype(np.float64) * np.repeat(scales.astype(np.float64), 128, axis=1)
     x = x.astype(np.float64)
     want = x @ w.T
     unit = np.abs(x).reshape(x.shape[0], groups, 128).max(axis=2) / 8355711.0
     off = 0.51 * np.repeat(unit, 128, axis=1) + np.abs(x) * (2.0 ** -22 + (groups + 6) * 2.0 ** -24)
-    bound = off @ np.abs(w).T
+    bound = off @ np.abs(w).T + floor
     diff = np.abs(got.astype(np.float64) - want)
     assert np.all(diff <= bound), f"max over bound {np.max(diff / np.maximum(bound, 1e-300)):.3g}"
 
@@ -94,6 +94,57 @@ def test_number_range(backend, case):
     check(got, x, codes, scales)
     if case == "zeros":
         assert not got[7].any()
+
+
+# Launches of 1 x 1, 1 x 2 (32 groups or more), 2 x 2 wave tiles, of K runs, and
+# a pair's; the last column of the block is ragged in each.
+SMALL_SHAPES = [(40, 200, 512), (300, 1300, 4096), (1030, 3300, 256), (20, 70, 2816)]
+
+
+@pytest.mark.parametrize("m,n,k", SMALL_SHAPES)
+@pytest.mark.parametrize("power", [-41, -104, -116, -120])
+def test_small_values(backend, power, m, n, k):
+    """Activations whose digit units, or units times scales, are below f32's
+    normal range: every row, then single rows and groups between ordinary ones.
+    A group's sum may itself be subnormal and round at 2^-149."""
+    say("i8 small", power, m, n, k)
+    floor = k // 128 * 2.0 ** -149
+    codes, scales = make_weights(n, k, "int8", 0x5EED0860)
+    x = convert.normal((m, k), 0xAC70860)
+    small = x * np.float32(2.0 ** power)
+    check(run_linear(backend, small, codes, scales), small, codes, scales, floor)
+    mixed = x.copy()
+    mixed[3::7] = small[3::7]
+    mixed[5, 128:256] = small[5, 128:256]
+    mixed[m - 1, :128] = small[m - 1, :128]
+    check(run_linear(backend, mixed, codes, scales), mixed, codes, scales, floor)
+
+
+def test_small_values_in_pairs(backend):
+    say("i8 small pair")
+    m, n, k = 70, 300, 1024
+    (ca, sa), (cb, sb) = (make_weights(n, k, "int8", 0x5EED0870 + i) for i in range(2))
+    x = convert.normal((m, k), 0xAC70870) * np.float32(2.0 ** -112)
+    x[::3] *= np.float32(2.0 ** 112)
+    a, b = upload_weights(backend, ca, sa), upload_weights(backend, cb, sb)
+    xb = backend.upload_f32(x.shape, x)
+    out_a, out_b = (backend.allocate_f32((m, n)) for _ in range(2))
+    backend.packed_linear_pair(out_a, out_b, xb, *a, *b)
+    check(backend.read(out_a), x, ca, sa, k // 128 * 2.0 ** -149)
+    check(backend.read(out_b), x, cb, sb, k // 128 * 2.0 ** -149)
+
+
+@pytest.mark.parametrize("x_power,scale_power", [(0, -116), (-60, -55), (60, -118), (-30, 80),
+                                                 (-100, 60)])
+def test_f32_scales_far_from_one(backend, x_power, scale_power):
+    say("i8 f32 scale range", x_power, scale_power)
+    m, n, k = 35, 200, 640
+    rng = np.random.default_rng(0x5EED0880)
+    codes = rng.integers(-127, 128, (n, k), dtype=np.int8).view(np.uint8)
+    scales = rng.uniform(0.01, 0.03, (n, k // 128)).astype(np.float32)
+    scales[1::2] *= np.float32(2.0 ** scale_power)
+    x = convert.normal((m, k), 0xAC70880) * np.float32(2.0 ** x_power)
+    check(run_linear(backend, x, codes, scales), x, codes, scales, k // 128 * 2.0 ** -149)
 
 
 def test_f32_scales(backend):
