@@ -18,7 +18,8 @@ namespace mfh {
 
 // 16 bytes per lane, from base + offset (uniform base, the lane's byte offset)
 // to the LDS bytes [lds, lds + 1024) of the wave.  The caller waits (vmcnt)
-// and synchronises before the bytes are read.
+// and synchronises before the bytes are read.  (m0 is the compiler's to reserve: it
+// sets it anew before each use of its own.)
 __device__ __forceinline__ void copy_to_lds(const uint8_t *base, uint32_t offset, uint32_t lds)
 {
     asm volatile("s_mov_b32 m0, %0\n\t"
@@ -26,7 +27,16 @@ __device__ __forceinline__ void copy_to_lds(const uint8_t *base, uint32_t offset
                  "global_load_lds_dwordx4 %1, %2"
                  :
                  : "s"(lds), "v"(offset), "s"(base)
-                 : "memory", "m0");
+                 : "memory");
+}
+
+// The lane, for code off the hot path: no register of the caller's stays live for
+// it.
+__device__ __forceinline__ uint32_t cold_lane()
+{
+    uint32_t lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+    return lane;
 }
 
 // A NaN that stands for the group's own code (0: a non-finite value, whose row

@@ -16,10 +16,14 @@
 //   block scale, and the levels' -1 enters as the accumulator's start value,
 //   minus the row's sum over the group.
 // - v_mfma_scale_f32_16x16x128_f8f6f4 multiplies exactly, applies both block
-//   scales and accumulates in f32; a 128-group is five of them, the smallest
-//   digit first.  The epilogue adds group_sum * scale in f32 (one FMA).
+//   scales and accumulates in f32; a 128-group is five of them, the largest
+//   digit first, which cancels the start value at once.  The epilogue adds group_sum * scale in f32 (one FMA).
 // - A row with a non-finite value gets NaN start values, so all of its
 //   outputs are NaN, as with a NaN or infinity in every dot.
+// - These are sums of true magnitudes (small ones keep their precision: the
+//   accumulators hold subnormals).  A group of a row with a run past 2^100 is
+//   written times 2^-64 and takes the range plan of digits.hpp: its start value is
+//   a code, and the second pass multiplies by signed levels, which need none.
 //
 // Bound and split.  FP6 x FP4 runs at four times the binary16 rate (measured
 // 8.2 against 2.27 PFLOP/s with eight waves per CU), so five passes cost 1.25
@@ -53,6 +57,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
+#include "digits.hpp"
 #include "kernels.hpp"
 
 namespace mfh {
@@ -75,6 +80,9 @@ constexpr uint32_t kDigitBytes = 64 * 24;
 constexpr uint32_t kSumsAt = kDigits * kDigitBytes;  // 16 f32: -(row sum)
 constexpr uint32_t kExpsAt = kSumsAt + 64;           // 64 bytes: block scales
 constexpr uint32_t kRecord = kExpsAt + 64;
+// A row's group with a run past 2^kLargeRun is written times 2^-kShift.
+constexpr int kLargeRun = 100, kShift = 64;
+constexpr uint32_t kShifted = 1;  // its start value's code
 // Records a block may read past the last row tile of the last group.
 constexpr uint32_t kMaxRowTiles = 2;
 
@@ -115,7 +123,11 @@ __global__ __launch_bounds__(kThreads) void mx_split_kernel(const float *__restr
     int e = 0;
     if (mx > 0.0f && !bad)
         frexpf(mx, &e);  // |x| < 2^e
-    e = e < -124 ? -124 : e;
+    int shift = 0;
+    const unsigned long long large = __ballot(e > kLargeRun);
+    if (__builtin_expect(large != 0, 0))
+        shift = (large >> i) & 0x0001000100010001ull ? kShift : 0;
+    e = max(e, shift - 124);
     // Operand slots 2t and 2t + 1 take even[t] and odd[t].  Slot order of the
     // weight nibbles: k = 0, 2, .., 14, 1, 3, .., 15 of each run of 16.
     v16f even, odd;
@@ -154,9 +166,10 @@ __global__ __launch_bounds__(kThreads) void mx_split_kernel(const float *__restr
     sum += __shfl_xor(sum, 32, 64);
     const unsigned long long any_bad = __ballot(bad);
     const bool row_bad = (any_bad >> i) & 0x0001000100010001ull;
-    out[kExpsAt + lane] = uint8_t(127 + e - 2);
+    out[kExpsAt + lane] = uint8_t(127 + e - 2 - shift);
     if (q == 0)
-        reinterpret_cast<float *>(out + kSumsAt)[i] = row_bad ? __builtin_nanf("") : float(-sum);
+        reinterpret_cast<float *>(out + kSumsAt)[i] =
+            row_bad ? nan_of(0) : shift ? nan_of(kShifted) : float(-sum);
 }
 
 struct MxArgs {
@@ -173,20 +186,6 @@ struct MxArgs {
     uint32_t tiles_n, tiles;   // output block tiles along n, and in all
     uint32_t chunks, chunk_groups;
 };
-
-// 16 bytes per lane, from base + offset (uniform base, the lane's byte offset)
-// to the LDS bytes [lds, lds + 1024) of the wave.  The caller waits (vmcnt)
-// and synchronises before the bytes are read.  Nothing else in this file uses
-// m0.
-__device__ __forceinline__ void copy_to_lds(const uint8_t *base, uint32_t offset, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "s_nop 0\n\t"
-                 "global_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds), "v"(offset), "s"(base)
-                 : "memory");
-}
 
 template <int S, Epilogue E, bool HALF, int TI, int TJ>
 __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
@@ -381,6 +380,76 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
     }
     if (grp < g_end)
         step(grp, std::integral_constant<int, 0>{});
+
+    // NaN totals (of rows that exist: the records past the last are no rows).
+    float nan = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+        if (mt0 + i < g.row_tiles) {
+#pragma unroll
+            for (int jt = 0; jt < TJ; ++jt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    nan += total[i][jt][r];
+        }
+    if (__builtin_expect(__any(nan != nan), 0)) {
+        // A tile at a time, straight from memory, on signed levels.
+        const uint32_t at = cold_lane(), ci = at & 15, cq = at >> 4;
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int jt = 0; jt < TJ; ++jt) {
+                if (mt0 + i >= g.row_tiles)
+                    continue;
+                v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                for (uint32_t gr = g_begin; gr < g_end; ++gr) {
+                    const uint8_t *rec = x_src + gr * x_step + i * kRecord;
+                    const v2u codes = *reinterpret_cast<const v2u *>(
+                        wptr[jt] + size_t(gr / 2) * 1024 + 16 * at + 8 * (gr & 1));
+                    v8i level = {};
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const unsigned w = ((codes[t / 2] ^ 0x80808080u) >> (2 * (t & 1))) &
+                                           0x33333333u;
+                        // Nibbles 0..3 to the FP4 values -0.5, 0, 0.5 and 1.
+                        const unsigned zero = ~(w | w >> 1) & 0x11111111u;
+                        level[t] = int((w - (zero ^ 0x11111111u)) | zero * 9);
+                    }
+                    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                    for (int d = kDigits - 1; d >= 0; --d) {
+                        const v4u lo =
+                            *reinterpret_cast<const v4u *>(rec + d * kDigitBytes + 16 * at);
+                        const v2u hi = *reinterpret_cast<const v2u *>(rec + d * kDigitBytes +
+                                                                      1024 + 8 * at);
+                        const v8i ad = {int(lo[0]), int(lo[1]), int(lo[2]), int(lo[3]),
+                                        int(hi[0]), int(hi[1]), 0, 0};
+                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                            ad, level, acc, 2, 4, 0, int(rec[kExpsAt + at]), 0,
+                            128 - kDigitBits * d);
+                    }
+                    const char *sp = sptr[jt] + (size_t(gr) * 16 + ci) * sizeof(Scale);
+                    float gs;
+                    if constexpr (HALF)
+                        gs = __half2float(*reinterpret_cast<const __half *>(sp));
+                    else
+                        gs = *reinterpret_cast<const float *>(sp);
+                    int gs_exp = 0;
+                    const float gs_frac = frexpf(gs, &gs_exp);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const uint32_t start =
+                            reinterpret_cast<const uint32_t *>(rec + kSumsAt)[4 * cq + r];
+                        if (start == kNanBits)
+                            sum[r] = nan_of(0);
+                        const int back = start == (kNanBits | kShifted) ? kShift : 0;
+                        sum[r] += ldexpf(acc[r] * gs_frac, gs_exp + back);
+                    }
+                }
+                total[i][jt] = sum;
+            }
+    }
 
 #pragma unroll
     for (int i = 0; i < TI; ++i)

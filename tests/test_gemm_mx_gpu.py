@@ -31,9 +31,9 @@ def reference(x, codes, scales):
     return x @ (level * scale).T, np.abs(x) @ ((np.abs(level) + 1.0) * np.abs(scale)).T
 
 
-def check(got, x, codes, scales):
+def check(got, x, codes, scales, floor=0.0):
     want, size = reference(x, codes, scales)
-    bound = (8 + scales.shape[1] / 2) * 2.0 ** -23 * size
+    bound = (8 + scales.shape[1] / 2) * 2.0 ** -23 * size + floor
     diff = np.abs(got.astype(np.float64) - want)
     assert np.all(diff <= bound), f"max over bound {np.max(diff / np.maximum(bound, 1e-300)):.3g}"
 
@@ -96,6 +96,57 @@ def test_number_range(backend, case):
         assert not got[7].any()
 
 
+# Launches of 1 x 1, 1 x 2 (32 groups or more), 2 x 2 and 2 x 4 wave tiles, and of
+# K runs, the odd one starting inside a 256-wide tile load; the last column of
+# the block is ragged in each.
+RANGE_SHAPES = [(40, 200, 512), (300, 1300, 4096), (1030, 1700, 256), (1025, 3300, 384),
+                (20, 70, 2816)]
+
+
+@pytest.mark.parametrize("m,n,k", RANGE_SHAPES)
+@pytest.mark.parametrize("power", [-61, -100, -116, -120, 99, 121, 124])
+def test_values_at_the_ends_of_the_range(backend, power, m, n, k):
+    """All rows, then single rows and groups between ordinary ones.  The large
+    ones meet sparse levels and small scales: group sums (of |x| and of 2 |x|)
+    that overflow f32 where the products of every output stay finite."""
+    say("mx range ends", power, m, n, k)
+    codes, scales = make_weights(n, k, "ternary", 0x5EED0760)
+    floor = k // 128 * 2.0 ** -149  # a group's sum may itself be subnormal
+    if power > 0:
+        rng = np.random.default_rng(0x5EED0761)
+        level = np.where(rng.random((n, k)) < 0.05, rng.integers(0, 3, (n, k)), 1)
+        codes = np.zeros((n, k // 4), np.uint8)
+        for i in range(4):
+            codes |= (level[:, i::4] << (2 * i)).astype(np.uint8)
+    x = convert.normal((m, k), 0xAC70760)
+    if power > 0:
+        x = np.abs(x)
+    far = x * np.float32(2.0 ** power)
+    assert np.isfinite(far).all()
+    check(run_linear(backend, far, codes, scales), far, codes, scales, floor)
+    mixed = x.copy()
+    mixed[3::7] = far[3::7]
+    mixed[5, 128:256] = far[5, 128:256]
+    mixed[m - 1, :128] = far[m - 1, :128]
+    mixed[6, 100:140] = far[6, 100:140]
+    check(run_linear(backend, mixed, codes, scales), mixed, codes, scales, floor)
+
+
+@pytest.mark.parametrize("power", [-112, 124])
+def test_ends_of_the_range_in_pairs(backend, power):
+    say("mx range pair", power)
+    m, n, k = 70, 300, 1024
+    (ca, sa), (cb, sb) = (make_weights(n, k, "ternary", 0x5EED0770 + i) for i in range(2))
+    x = convert.normal((m, k), 0xAC70770)
+    x[::3] *= np.float32(2.0 ** power)
+    a, b = upload_weights(backend, ca, sa), upload_weights(backend, cb, sb)
+    xb = backend.upload_f32(x.shape, x)
+    out_a, out_b = (backend.allocate_f32((m, n)) for _ in range(2))
+    backend.packed_linear_pair(out_a, out_b, xb, *a, *b)
+    check(backend.read(out_a), x, ca, sa, k // 128 * 2.0 ** -149)
+    check(backend.read(out_b), x, cb, sb, k // 128 * 2.0 ** -149)
+
+
 def test_reserved_code_and_f32_scales(backend):
     say("mx reserved code")
     m, n, k = 35, 100, 640
@@ -103,6 +154,8 @@ def test_reserved_code_and_f32_scales(backend):
     codes = rng.integers(0, 256, (n, k // 4), dtype=np.uint8)  # code 3 is level +2
     scales = rng.uniform(0.01, 0.03, (n, k // 128)).astype(np.float32)  # not binary16 values
     x = convert.normal((m, k), 0xAC70730)
+    check(run_linear(backend, x, codes, scales), x, codes, scales)
+    x[::2] *= np.float32(2.0 ** -110)
     check(run_linear(backend, x, codes, scales), x, codes, scales)
 
 
