@@ -1,25 +1,24 @@
-// Prefill attention at head width 64 on binary16 matrix cores, f32-exact
-// operands split in halves.
+// Prefill attention at head width 64 on bfloat16 matrix cores, f32 operands split
+// in three parts.
 //
-// Flash-style causal GQA for many (token, query head) pairs.  A block of
-// kWaves waves serves one key/value head and kRows query rows: `tile_tokens`
-// consecutive tokens times the group's query heads (row r is token t0 + r /
-// group, query head r % group of the key/value head); each wave owns 16 rows.
-// Key and value rows stream through LDS in kKeys-key tiles that every row of
-// the block shares.
+// Flash-style causal GQA for many (token, query head) pairs.  A block serves one
+// key/value head and kRows query rows: `tile_tokens` consecutive tokens times the
+// group's query heads (row r is token t0 + r / group, query head r % group of the
+// key/value head).  Its two teams of kWaves waves, 16 rows each, take the kKeys-key
+// tiles in turn, each through LDS tiles of its own that every row of the team
+// shares, and the first team adds the second's rows to its own in the end.
 //
-// Exactness plan.  Every operand is a power of two times hi + lo binary16
-// halves: a query row by its own largest magnitude, a key tile by the tile's,
-// a value tile by the largest seen so far (the output accumulators are
-// rescaled when it grows), probabilities by 2^7 (they stay below 2^8).  The
-// largest magnitude sits below 2^15, so a value keeps 22 bits down to 2^-18 of it and an absolute
-// error of 2^-40 of it below that.  Products are exact in f32; lo * lo, below
-// 2^-22 of each term, is dropped.  Scores, the softmax and all sums are f32.
-// Where a key or value of a block's range is infinite, or a wave's query is not
-// finite, the rows are computed again on v_mfma_f32_16x16x4_f32 from the f32
-// values, so infinities act as in f32 arithmetic (NaN does in both halves).  A
-// key the causal mask hides gets probability zero; a non-finite value row later
-// in the same tile still reaches the earlier rows (0 * NaN), where the
+// Exactness plan.  Every query, key, value and probability is the sum of three
+// bfloat16 parts that hold all 24 bits (bfloat16 has the exponents of f32, so no
+// scale is shared between elements).  Of the nine products of parts the three
+// below 2^-23 of a term are left out; products are exact in f32.  Scores, the
+// softmax and all sums are f32, and a tile's share of the output is summed by
+// itself before it is added.  Where the largest of eight staged values is past
+// 2^60 (an infinity, or one whose parts or products could overflow) or below 2^-100
+// (whose parts are subnormal), or eight of a wave's query are, the rows are
+// computed again on v_mfma_f32_16x16x4_f32 from the f32 values (NaN acts alike in
+// both).  A key the causal mask hides gets probability zero; a non-finite value row
+// later in the same tile still reaches the earlier rows (0 * NaN), where the
 // reference skips it (attention_convolution.rs:90-170).
 //
 // Per tile, S^T = K Q^T leaves row j of a wave in lane column j: lane 16q + j
@@ -30,16 +29,18 @@
 // in that key order.
 //
 // LDS holds each operand in 16-byte chunks, [16-row tile][chunk][row], so a
-// wave's operand read is one contiguous KB; the row index is swizzled to spread
-// the staging writes over the banks.
+// wave's operand read is one contiguous KB; the row index is swizzled so that the
+// staging writes of 16 (keys) and 32 (values) lanes fall on distinct banks.
 //
-// Bound.  Per wave and tile 48 MFMAs (768 cycles) against about 290 vector
-// instructions of softmax and splitting, the two overlapping across the four
-// waves of a SIMD; the causal triangle leaves 2.4 of them busy on average.
-// 2048 tokens, 32 / 8 heads: 101 us per call with the cache append, against 227
-// for the fp32 matrix cores this replaces (128 MFMAs of 32 cycles per tile);
-// error against 64-bit sums 2.6e-7 (before: 4.0e-7).  One 16-wave block per CU
-// whose halves take tiles in turn measured 104 us.
+// Bound.  Per wave and tile 96 MFMAs (1536 cycles) and about 350 vector
+// instructions (1400 cycles) of softmax and splitting, which hardly overlap: they
+// take 80 % of the time.  2048 tokens, 32 / 8 heads: 119 us per call with the cache
+// append, 227 on the fp32 matrix cores (128 MFMAs of 32 cycles per tile), 100 on
+// binary16 hi + lo halves with shared scales, which lost small values beside large
+// ones; error against 64-bit sums 1.8e-7 (fp32 matrix cores 4.0e-7, halves 2.6e-7;
+// summing the tiles in one chain 3.2e-7).  One team of eight waves per block, two
+// blocks per CU, measured 136 us (the causal triangle leaves a CU one long block);
+// two teams of four waves with 32 rows each 126.
 #include <algorithm>
 
 #include <hip/hip_runtime.h>
@@ -49,53 +50,34 @@
 namespace mfh {
 namespace {
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v2f __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
-constexpr int kWaves = 8;  // of 16 rows each
-constexpr uint32_t kThreads = 64 * kWaves;
+constexpr int kTeams = 2;
+constexpr int kWaves = 8;  // per team, of 16 rows each
+constexpr uint32_t kThreads = 64 * kWaves;  // per team
 constexpr uint32_t kRows = 16 * kWaves;
 constexpr uint32_t kKeys = 64;
 constexpr uint32_t kDim = 64;
-constexpr uint32_t kPlane = kKeys * kDim * 2;  // one half of one operand tile
-constexpr int kTop = 15;                       // scaled magnitudes stay below 2^kTop
+constexpr int kParts = 3;                      // bfloat16 parts of an operand
+constexpr uint32_t kPlane = kKeys * kDim * 2;  // one part of one operand tile
 constexpr int kSlack = 8;                      // p stays below 2^kSlack
-constexpr int kMinExponent = -90;              // smaller values keep this scale
+// Magnitudes whose parts are normal and whose products are finite.
+constexpr float kSmallest = 0x1p-100f, kLargest = 0x1p60f;
 
 // Byte offset of row `row`'s 16-byte chunk `chunk` (of 8) in a plane.
 __device__ __forceinline__ uint32_t key_at(uint32_t row, uint32_t chunk)
 {
-    return (row >> 4) * 2048 + chunk * 256 + (((row & 15) ^ ((chunk & 1) << 3)) << 4);
+    return (row >> 4) * 2048 + chunk * 256 + (((row & 15) ^ (2 * chunk)) << 4);
 }
 __device__ __forceinline__ uint32_t value_at(uint32_t dim, uint32_t chunk)
 {
     return (dim >> 4) * 2048 + chunk * 256 + (((dim & 15) ^ ((dim >> 4) & 1)) << 4);
 }
-
-__device__ __forceinline__ uint32_t magnitude(float x)
-{
-    return __builtin_bit_cast(uint32_t, x) & 0x7fffffffu;
-}
-
-constexpr uint32_t kInfBits = 0x7f800000u;
-
-// The exponent e with every magnitude pattern up to `bits` (finite) below 2^e.
-__device__ __forceinline__ int exponent_of(uint32_t bits)
-{
-    const int e = int(bits >> 23) - 126;
-    return e < kMinExponent ? kMinExponent : e;
-}
-
-// 2^e, -126 <= e <= 127.
-__device__ __forceinline__ float power_of_two(int e)
-{
-    return __builtin_bit_cast(float, uint32_t(e + 127) << 23);
-}
-
-__device__ __forceinline__ uint32_t larger(uint32_t a, uint32_t b) { return a > b ? a : b; }
 
 // max(a, |b|, |c|); NaN operands are ignored.
 __device__ __forceinline__ float max3_abs(float a, float b, float c)
@@ -105,19 +87,16 @@ __device__ __forceinline__ float max3_abs(float a, float b, float c)
     return r;
 }
 
-// Maximum over the wave of a magnitude's bits: DPP within the 16-lane rows,
-// then row swaps.
-__device__ __forceinline__ uint32_t wave_max_bits(float m)
+// Whether x's largest magnitude is neither zero nor in the range of the parts.
+template <int N, typename F>
+__device__ __forceinline__ bool out_of_range(const F &x)
 {
-    uint32_t v = __float_as_uint(m);
-    v = larger(v, uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true)));   // xor 1
-    v = larger(v, uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true)));   // xor 2
-    v = larger(v, uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x141, 0xF, 0xF, true)));  // half mirror
-    v = larger(v, uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x140, 0xF, 0xF, true)));  // mirror
-    const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    v = larger(a[0], a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return larger(b[0], b[1]);
+    static_assert(N % 2 == 0, "pairs");
+    float most = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; i += 2)
+        most = max3_abs(most, x[i], x[i + 1]);
+    return most > kLargest || (most < kSmallest && most != 0.0f);
 }
 
 // Maximum and sum over a row's four lanes (q = 0..3).
@@ -140,36 +119,71 @@ __device__ __forceinline__ float quad_sum(float v)
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// hi + lo of x * scale.  (Adding zero keeps both on the mixed-precision FMA,
-// which rounds straight to binary16.)
-template <int N, typename F, typename H>
-__device__ __forceinline__ void split(const F &x, float scale, H &hi, H &lo)
+// x[0..N) as N / 2 dwords of bfloat16 pairs in each of three parts: every part is
+// the nearest bfloat16 of what the ones before it left, and the three hold all 24
+// bits.
+template <int N, typename F, typename P>
+__device__ __forceinline__ void split(const F &x, P &hi, P &mid, P &lo)
 {
+    auto nearest = [](float a, float b) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2b));
+    };
+    auto first = [](uint32_t pair) { return __uint_as_float(pair << 16); };
+    auto second = [](uint32_t pair) { return __uint_as_float(pair & 0xffff0000u); };
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        hi[i] = _Float16(fmaf(x[i], scale, 0.0f));
-        lo[i] = _Float16(fmaf(x[i], scale, -float(hi[i])));
+    for (int i = 0; i < N / 2; ++i) {
+        float a = x[2 * i], b = x[2 * i + 1];
+        hi[i] = nearest(a, b);
+        a -= first(hi[i]);
+        b -= second(hi[i]);
+        mid[i] = nearest(a, b);
+        a -= first(mid[i]);
+        b -= second(mid[i]);
+        lo[i] = nearest(a, b);
     }
 }
 
-__global__ __launch_bounds__(kThreads, 4) void gqa_flash_split_kernel(
+// c + a b without the products below 2^-24 of a term, smallest first.
+struct Parts {
+    v4u hi, mid, lo;
+};
+__device__ __forceinline__ v4f multiply_add(const v4u &a, const v4u &b, const v4f &c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8b, a),
+                                                   __builtin_bit_cast(v8b, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ v4f multiply_add(const Parts &a, const Parts &b, v4f c)
+{
+    c = multiply_add(a.lo, b.hi, c);
+    c = multiply_add(a.hi, b.lo, c);
+    c = multiply_add(a.mid, b.mid, c);
+    c = multiply_add(a.mid, b.hi, c);
+    c = multiply_add(a.hi, b.mid, c);
+    return multiply_add(a.hi, b.hi, c);
+}
+
+__global__ __launch_bounds__(kTeams * kThreads, 4) void gqa_flash_split_kernel(
     float *__restrict__ out, const float *__restrict__ query, const float *__restrict__ key_cache,
     const float *__restrict__ value_cache, GqaShape g, uint32_t tile_tokens, uint32_t token_tiles,
-    bool paired, uint32_t ranges, uint32_t range_tiles, float *__restrict__ records)
+    uint32_t ranges, uint32_t range_tiles, float *__restrict__ records)
 {
-    __shared__ __align__(1024) uint8_t lds[2][4 * kPlane];  // K hi, K lo, V^T hi, V^T lo
-    __shared__ uint32_t wave_bits[2][2][kWaves];
+    // Per team the parts of a key tile and of a transposed value tile; in the end
+    // the second team's accumulators.
+    constexpr uint32_t kTile = kParts * kPlane;
+    __shared__ __align__(1024) uint8_t lds[kTeams][2 * kTile];
+    // The parts of the rows' queries, [part][step].
+    __shared__ __align__(1024) v4u q_lds[kParts][2][kThreads];
 
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t tid = threadIdx.x % kThreads, lane = tid & 63;
+    const uint32_t team = __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t *const k_lds = lds[team], *const v_lds = k_lds + kTile;
     const uint32_t q = lane >> 4, j = lane & 15;
     const uint32_t kv_heads = g.key_value_heads, group = g.group;
     const uint32_t kv_head = blockIdx.x % kv_heads;
-    const uint32_t range = blockIdx.x / kv_heads % ranges, nth = blockIdx.x / kv_heads / ranges;
-    // Longest token tiles (most keys) first; where the whole grid is resident,
-    // its second half runs shortest first, beside the first half's long ones.
-    const uint32_t half = (token_tiles + 1) / 2;
-    const uint32_t tile = paired && nth >= half ? nth - half : token_tiles - 1 - nth;
+    const uint32_t range = blockIdx.x / kv_heads % ranges;
+    // Longest token tiles (most keys) first: a CU that is done takes a shorter one.
+    const uint32_t tile = token_tiles - 1 - blockIdx.x / kv_heads / ranges;
     const uint32_t start = uint32_t(g.initial_len), tokens = uint32_t(g.tokens);
     const uint32_t t0 = tile * tile_tokens;
     const uint32_t t_end = t0 + tile_tokens < tokens ? t0 + tile_tokens : tokens;
@@ -184,188 +198,161 @@ __global__ __launch_bounds__(kThreads, 4) void gqa_flash_split_kernel(
     const uint32_t token = t0 + row / group;
     const uint32_t head = kv_head * group + row % group;
     const bool valid = row < tile_tokens * group && token < tokens;
-    const uint32_t last = valid ? start + token : k_end - 1;  // last visible key
-    const uint32_t wave_first = start + t0 + 16 * wave / group;         // smallest `last`
-    const uint32_t wave_last = start + t0 + (16 * wave + 15) / group;  // largest stored `last`
+    // The last visible key, less the lane's first one of 16.
+    const int reach = int(valid ? start + token : k_end - 1) - int(4 * q);
+    const uint32_t wave_first = start + t0 + 16 * wave / group;         // smallest last key
+    const uint32_t wave_last = start + t0 + (16 * wave + 15) / group;  // largest stored one
     const float *const q_row = query + (size_t(valid ? token : 0) * g.query_heads + head) * kDim;
 
     // Q^T operand: dimensions 32s + 8q + e of the row at step s.
-    v8h qh[2], ql[2];
-    float row_scale;  // of the scores: 1 / sqrt(d), log2(e) and the row's power of two
-    bool q_bad;
-    constexpr float kLog2e = 1.44269504088896341f;
-    {
-        float f[2][8];
-        uint32_t bits = 0;
+    bool q_bad = false;  // of the wave
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+    for (int s = 0; s < 2; ++s) {
+        float f[8];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const v4f v = valid ? *reinterpret_cast<const v4f *>(q_row + 32 * s + 8 * q + 4 * h)
-                                    : v4f{0, 0, 0, 0};
+        for (int h = 0; h < 2; ++h) {
+            const v4f v = valid ? *reinterpret_cast<const v4f *>(q_row + 32 * s + 8 * q + 4 * h)
+                                : v4f{0, 0, 0, 0};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    f[s][4 * h + e] = v[e];
-                    bits = larger(bits, magnitude(v[e]));
-                }
-            }
-        bits = larger(bits, __shfl_xor(bits, 16, 64));
-        bits = larger(bits, __shfl_xor(bits, 32, 64));
-        q_bad = __any(bits >= kInfBits);
-        const int e = bits >= kInfBits ? 0 : exponent_of(bits);
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            split<8>(f[s], power_of_two(kTop - e), qh[s], ql[s]);
-        row_scale = g.scale * kLog2e * power_of_two(e - kTop);
+            for (int e = 0; e < 4; ++e)
+                f[4 * h + e] = v[e];
+        }
+        q_bad |= __any(out_of_range<8>(f));
+        if (team == 0) {
+            Parts p;
+            split<8>(f, p.hi, p.mid, p.lo);
+            q_lds[0][s][tid] = p.hi;
+            q_lds[1][s][tid] = p.mid;
+            q_lds[2][s][tid] = p.lo;
+        }
     }
+    constexpr float kLog2e = 1.44269504088896341f;
+    const float unit = g.scale * kLog2e;
 
     // Staging: a thread loads chunk `tid % 8` of key `tid / 8`, and dimensions
-    // 2b, 2b + 1 of keys 4a..4a + 3.
+    // 2b, 2b + 1 of keys 4a..4a + 3.  Those keys are the low (a % 8 < 4) or high
+    // half of the chunk of lane block a % 4 at 32-key step a / 8; a wave stores both
+    // halves of one chunk.
     const uint32_t k_key = tid / 8, k_chunk = tid % 8;
-    const uint32_t v_quad = tid / 32, v_pair = tid % 32;
+    const uint32_t v_high = (tid >> 4) & 1, v_pair = (tid & 15) | ((tid >> 5) & 1) << 4;
+    const uint32_t v_key = 4 * (wave / 4 * 8 + v_high * 4 + wave % 4);
     v4f kr[2];
     v2f vr[4];
     // Rows past the end repeat the last one: the mask hides their scores, and
     // as values they meet probability zero.
     const uint32_t row_bytes = uint32_t(kv_width) * 4;
-    auto stage_load = [&](uint32_t n) {
-        const uint32_t k0 = n * kKeys, most = k_end - 1 - k0;
+    const uint32_t k_row = k_key * row_bytes, v_row = v_key * row_bytes;
+    auto load_keys = [&](uint32_t n) {
+        const uint32_t k0 = n * kKeys, most = min(k_end - 1 - k0, kKeys - 1) * row_bytes;
         const char *const kt = reinterpret_cast<const char *>(keys + k0 * kv_width);
+        const uint32_t at = min(k_row, most) + 32 * k_chunk;
+        kr[0] = *reinterpret_cast<const v4f *>(kt + at);
+        kr[1] = *reinterpret_cast<const v4f *>(kt + at + 16);
+    };
+    auto load_values = [&](uint32_t n) {
+        const uint32_t k0 = n * kKeys, most = min(k_end - 1 - k0, kKeys - 1) * row_bytes;
         const char *const vt = reinterpret_cast<const char *>(values + k0 * kv_width);
-        const uint32_t k_off = min(k_key, most) * row_bytes + 32 * k_chunk;
-        kr[0] = *reinterpret_cast<const v4f *>(kt + k_off);
-        kr[1] = *reinterpret_cast<const v4f *>(kt + k_off + 16);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            vr[i] = *reinterpret_cast<const v2f *>(
-                vt + min(4 * v_quad + i, most) * row_bytes + 8 * v_pair);
-    };
-
-    // What a staged tile's halves are scaled by.
-    struct Scales {
-        int v_exp = kMinExponent;  // values: 2^(kTop - v_exp), growing with the tiles
-        float k_unit = 1.0f;       // keys: their power of two
-        bool bad = false;          // an infinity: nothing is staged
-    };
-    auto publish = [&](uint32_t slot, float a, float b) {
-        const uint32_t a_bits = wave_max_bits(a), b_bits = wave_max_bits(b);
-        if (lane == 0) {
-            wave_bits[slot][0][wave] = a_bits;
-            wave_bits[slot][1][wave] = b_bits;
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t at = min(v_row + i * row_bytes, most) + 8 * v_pair;
+            vr[i] = *reinterpret_cast<const v2f *>(vt + at);
         }
     };
-    auto block_max = [&](uint32_t slot, uint32_t which) {
-        uint32_t v = 0;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w)
-            v = larger(v, wave_bits[slot][which][w]);
-        return uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
-    };
-    // The loaded tile's largest magnitudes (before the barrier) ...
-    auto stage_max = [&](uint32_t slot) {
-        float km = 0.0f, vm = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            km = max3_abs(km, kr[i / 2][2 * (i % 2)], kr[i / 2][2 * (i % 2) + 1]);
-            vm = max3_abs(vm, vr[i][0], vr[i][1]);
-        }
-        publish(slot, km, vm);
-    };
-    // ... and its halves (after it).
-    auto stage_store = [&](uint32_t slot, Scales &t) {
-        const uint32_t k_bits = block_max(slot, 0), v_bits = block_max(slot, 1);
-        t.bad = larger(k_bits, v_bits) >= kInfBits;
-        if (t.bad)
-            return;
-        const int ve = exponent_of(v_bits);
-        t.v_exp = ve > t.v_exp ? ve : t.v_exp;
-        const int ke = exponent_of(k_bits);
-        t.k_unit = power_of_two(ke - kTop);
-        const float ks = power_of_two(kTop - ke), vs = power_of_two(kTop - t.v_exp);
-        uint8_t *const k_hi = lds[slot], *const v_hi = k_hi + 2 * kPlane;
-        v8h hi, lo;
+    bool bad = false;  // a value out of the parts' range was staged
+    auto store_keys = [&] {
         float f[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             f[i] = kr[i / 4][i % 4];
-        split<8>(f, ks, hi, lo);
-        *reinterpret_cast<v8h *>(k_hi + key_at(k_key, k_chunk)) = hi;
-        *reinterpret_cast<v8h *>(k_hi + kPlane + key_at(k_key, k_chunk)) = lo;
-        // Keys 4a..4a + 3 of 32-key step t are the low (a % 8 < 4) or high
-        // half of the chunk of lane block a % 4.
-        const uint32_t chunk = v_quad / 8 * 4 + v_quad % 4, high = v_quad % 8 / 4 * 8;
+        bad |= out_of_range<8>(f);
+        Parts p;
+        split<8>(f, p.hi, p.mid, p.lo);
+        uint8_t *const at = k_lds + key_at(k_key, k_chunk);
+        *reinterpret_cast<v4u *>(at) = p.hi;
+        *reinterpret_cast<v4u *>(at + kPlane) = p.mid;
+        *reinterpret_cast<v4u *>(at + 2 * kPlane) = p.lo;
+    };
+    auto store_values = [&] {
+        const float all[8] = {vr[0][0], vr[0][1], vr[1][0], vr[1][1],
+                              vr[2][0], vr[2][1], vr[3][0], vr[3][1]};
+        bad |= out_of_range<8>(all);
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
             const float x[4] = {vr[0][d], vr[1][d], vr[2][d], vr[3][d]};
-            v4h vh, vl;
-            split<4>(x, vs, vh, vl);
-            const uint32_t at = value_at(2 * v_pair + d, chunk) + high;
-            *reinterpret_cast<v4h *>(v_hi + at) = vh;
-            *reinterpret_cast<v4h *>(v_hi + kPlane + at) = vl;
+            v2u hi, mid, lo;
+            split<4>(x, hi, mid, lo);
+            uint8_t *const at = v_lds + value_at(2 * v_pair + d, wave) + 8 * v_high;
+            *reinterpret_cast<v2u *>(at) = hi;
+            *reinterpret_cast<v2u *>(at + kPlane) = mid;
+            *reinterpret_cast<v2u *>(at + 2 * kPlane) = lo;
         }
+    };
+    auto parts_at = [](const uint8_t *plane) {
+        return Parts{*reinterpret_cast<const v4u *>(plane),
+                     *reinterpret_cast<const v4u *>(plane + kPlane),
+                     *reinterpret_cast<const v4u *>(plane + 2 * kPlane)};
     };
 
     v4f o[4];
+    float m, l;  // m in log2 units
+    auto clear = [&] {
+        m = -__builtin_inff();
+        l = 0.0f;
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-        o[u] = v4f{0, 0, 0, 0};
-    int o_exp = kMinExponent;  // the value scale of the wave's accumulators
-    float m = -__builtin_inff(), l = 0.0f;  // m in log2 units
+        for (int u = 0; u < 4; ++u)
+            o[u] = v4f{0, 0, 0, 0};
+    };
+    clear();
     // The block's key tiles.
     const uint32_t tiles = (k_end + kKeys - 1) / kKeys;
     const uint32_t begin = range * range_tiles;
     const uint32_t end = begin + range_tiles < tiles ? begin + range_tiles : tiles;
-    Scales next;
-    if (begin < end) {
-        stage_load(begin);
-        stage_max(begin & 1);
-        __syncthreads();
-        stage_store(begin & 1, next);
-        if (begin + 1 < end)
-            stage_load(begin + 1);
+    if (begin + team < end) {
+        load_keys(begin + team);
+        load_values(begin + team);
+        store_keys();
     }
-    // Per tile one barrier: behind it the tile's halves are complete and the
-    // buffer of the tile before is free, so the next tile (in registers since
-    // the last one) is split into it and the one after requested while this one
-    // is multiplied.
-    for (uint32_t n = begin; n < end; ++n) {
+    // The teams take the key tiles in turn.  Per tile two barriers: behind the first
+    // the tile's keys are complete and the values of the tile before are free, behind
+    // the second the tile's values are complete and its keys are free.  The values
+    // (the next keys) to store there were requested half a tile earlier.
+    for (uint32_t first = begin; first < end; first += kTeams) {
+        const uint32_t n = first + team, next = n + kTeams;
         const uint32_t k0 = n * kKeys;
-        const Scales cur = next;
-        const uint8_t *const k_hi = lds[n & 1], *const v_hi = k_hi + 2 * kPlane;
-        if (n + 1 < end)
-            stage_max((n + 1) & 1);
+        const bool active = n < end && k0 <= wave_last && !q_bad;
         __syncthreads();
-        if (cur.bad)
-            break;
-        if (n + 1 < end)
-            stage_store((n + 1) & 1, next);
-        if (n + 2 < end)
-            stage_load(n + 2);
-        if (k0 <= wave_last && !q_bad) {
+        if (n < end)
+            store_values();
+        if (next < end)
+            load_keys(next);
+        v4f s[4];
+        if (active) {
             // S^T = K Q^T.
-            v4f s[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                v4f acc = {0, 0, 0, 0};
+            for (int c = 0; c < 4; ++c)
+                s[c] = v4f{0, 0, 0, 0};
 #pragma unroll
-                for (int st = 0; st < 2; ++st) {
-                    const uint32_t at = key_at(16 * c + j, 4 * st + q);
-                    const v8h kh = *reinterpret_cast<const v8h *>(k_hi + at);
-                    const v8h kl = *reinterpret_cast<const v8h *>(k_hi + kPlane + at);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[st], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[st], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[st], acc, 0, 0, 0);
-                }
-                s[c] = acc;
+            for (int st = 0; st < 2; ++st) {
+                const Parts qp = {q_lds[0][st][tid], q_lds[1][st][tid], q_lds[2][st][tid]};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    s[c] = multiply_add(parts_at(k_lds + key_at(16 * c + j, 4 * st + q)), qp,
+                                        s[c]);
             }
-            const float unit = fminf(fmaxf(row_scale * cur.k_unit, __FLT_MIN__), __FLT_MAX__);
+        }
+        __syncthreads();
+        if (next < end) {
+            store_keys();
+            load_values(next);
+        }
+        if (active) {
             // Causal mask, online softmax over the row's four lanes.
             if (k0 + kKeys - 1 > wave_first || k0 + kKeys > k_end) {
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        if (k0 + 16 * c + 4 * q + r > last)
+                        if (int(k0 + 16 * c + r) > reach)
                             s[c][r] = -__builtin_inff();
             }
             // The reference m of the exponents follows the running maximum
@@ -378,67 +365,55 @@ __global__ __launch_bounds__(kThreads, 4) void gqa_flash_split_kernel(
                 for (int r = c == 0 ? 1 : 0; r < 4; ++r)
                     mx = fmaxf(mx, s[c][r]);
             mx = quad_max(mx) * unit;
-            const int shrink = o_exp - cur.v_exp;
-            if (__any(mx > m + kSlack) || shrink != 0) {
+            if (__any(mx > m + kSlack)) {
                 // A row without a visible key so far keeps m = -inf, l = 0.
                 const float m_new = fmaxf(m, mx);
                 const float alpha =
                     m_new == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
                 m = m_new;
                 l *= alpha;
-                const float rescale = alpha * (shrink < -126 ? 0.0f : power_of_two(shrink));
-                o_exp = cur.v_exp;
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
-                    o[u] *= rescale;
+                    o[u] *= alpha;
             }
             const float m_ref = m == -__builtin_inff() ? 0.0f : m;
-            v8h ph[2], pl[2];
+            Parts p[2];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                float p[4];
+                v2u hi, mid, lo;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    p[r] = __builtin_amdgcn_exp2f(fmaf(s[c][r], unit, -m_ref));
-                    l += p[r];
-                    s[c][r] = p[r];
+                    s[c][r] = __builtin_amdgcn_exp2f(fmaf(s[c][r], unit, -m_ref));
+                    l += s[c][r];
                 }
-                v4h hi, lo;
-                split<4>(p, power_of_two(kTop - kSlack), hi, lo);
+                split<4>(s[c], hi, mid, lo);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    ph[c / 2][4 * (c % 2) + r] = hi[r];
-                    pl[c / 2][4 * (c % 2) + r] = lo[r];
+                for (int r = 0; r < 2; ++r) {
+                    p[c / 2].hi[2 * (c % 2) + r] = hi[r];
+                    p[c / 2].mid[2 * (c % 2) + r] = mid[r];
+                    p[c / 2].lo[2 * (c % 2) + r] = lo[r];
                 }
             }
-            // O^T += V^T P^T.
+            // O^T += V^T P^T, the tile's sums added whole.
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < 4; ++u) {
+                v4f sum = {0, 0, 0, 0};
 #pragma unroll
-                for (int st = 0; st < 2; ++st) {
-                    const uint32_t at = value_at(16 * u + j, 4 * st + q);
-                    const v8h vh = *reinterpret_cast<const v8h *>(v_hi + at);
-                    const v8h vl = *reinterpret_cast<const v8h *>(v_hi + kPlane + at);
-                    o[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[st], o[u], 0, 0, 0);
-                    o[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[st], o[u], 0, 0, 0);
-                    o[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[st], o[u], 0, 0, 0);
-                }
+                for (int st = 0; st < 2; ++st)
+                    sum = multiply_add(parts_at(v_lds + value_at(16 * u + j, 4 * st + q)), p[st],
+                                       sum);
+                o[u] += sum;
+            }
         }
     }
-    // The accumulators carry the scales of p and of the values.
-    float unscale = power_of_two(o_exp - 2 * kTop + kSlack);
-    if (next.bad || q_bad) {
-        // An infinity among the range's keys or values, or a non-finite query
-        // of this wave: the rows over again in f32, straight from memory.
-        unscale = 1.0f;
-        m = -__builtin_inff();
-        l = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            o[u] = v4f{0, 0, 0, 0};
-        const float unit = g.scale * kLog2e;
+    // (A barrier, so the tiles are free.)
+    if (__syncthreads_or(bad) || q_bad) {
+        // A key or value of the range, or a query of this wave, that the parts do
+        // not serve: the rows over again in f32, straight from memory.
+        clear();
 #pragma unroll 1
-        for (uint32_t k0 = begin * kKeys; k0 < end * kKeys && k0 <= wave_last; k0 += 16) {
+        for (uint32_t k0 = begin * kKeys + 16 * team; k0 < end * kKeys && k0 <= wave_last;
+             k0 += 16 * kTeams) {
             // 16 keys: scores of key 4q + r, operand key j.
             v4f s = {0, 0, 0, 0};
             const float *const kp = keys + size_t(min(k0 + j, k_end - 1)) * kv_width + 4 * q;
@@ -453,7 +428,7 @@ __global__ __launch_bounds__(kThreads, 4) void gqa_flash_split_kernel(
             float mx = -__builtin_inff();
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                s[r] = k0 + 4 * q + r > last ? -__builtin_inff() : s[r] * unit;
+                s[r] = int(k0 + r) > reach ? -__builtin_inff() : s[r] * unit;
                 mx = fmaxf(mx, s[r]);
             }
             const float m_new = fmaxf(m, quad_max(mx));
@@ -476,6 +451,29 @@ __global__ __launch_bounds__(kThreads, 4) void gqa_flash_split_kernel(
             }
         }
     }
+    // The second team hands its rows to the first.
+    static_assert(kThreads * (4 * 16 + 2 * 4) <= sizeof(lds), "the teams' exchange");
+    v4f *const o_lds = reinterpret_cast<v4f *>(lds[0]) + tid;
+    float *const ml_lds = reinterpret_cast<float *>(lds[0] + 4 * 16 * kThreads) + tid;
+    if (team != 0) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            o_lds[u * kThreads] = o[u];
+        ml_lds[0] = m;
+        ml_lds[kThreads] = l;
+    }
+    __syncthreads();
+    if (team != 0)
+        return;
+    const float m_other = ml_lds[0], m_new = fmaxf(m, m_other);
+    const float m_ref = m_new == -__builtin_inff() ? 0.0f : m_new;
+    const float w = __builtin_amdgcn_exp2f(m - m_ref);
+    const float w_other = __builtin_amdgcn_exp2f(m_other - m_ref);
+    m = m_new;
+    l = l * w + ml_lds[kThreads] * w_other;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        o[u] = o[u] * w + o_lds[u * kThreads] * w_other;
     l = quad_sum(l);  // each lane holds its own keys' share
     if (!valid)
         return;
@@ -491,7 +489,7 @@ __global__ __launch_bounds__(kThreads, 4) void gqa_flash_split_kernel(
         for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                rec[2 + 16 * u + 4 * q + e] = o[u][e] * unscale;
+                rec[2 + 16 * u + 4 * q + e] = o[u][e];
         return;
     }
     float *const o_row = out + pair * kDim;
@@ -500,7 +498,7 @@ __global__ __launch_bounds__(kThreads, 4) void gqa_flash_split_kernel(
         v4f r;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            r[e] = o[u][e] / l * unscale;
+            r[e] = o[u][e] / l;
         *reinterpret_cast<v4f *>(o_row + 16 * u + 4 * q) = r;
     }
 }
@@ -536,13 +534,14 @@ struct Grid {
     uint32_t tile_tokens, token_tiles, ranges, range_tiles;
 };
 
-// Blocks the CUs hold at once, two each (128 registers, 64 KB of LDS).
-constexpr uint32_t kResident = 512;
+// Blocks the CUs hold at once: one each.
+constexpr uint32_t kResident = 256;
 
-// A launch that leaves most CUs idle cuts its keys into ranges of at least four
-// tiles, whose records a second launch merges: 64 tokens over 2000 keys (32 / 8
-// heads) 112 -> 24 us, 1024 over 1024 (16 / 4) 111 -> 57.  Fuller launches lose
-// by the records' traffic (2048 tokens 101 unsplit, 141 in two ranges).
+// A launch that leaves half of the CUs idle cuts its keys into ranges of at least
+// four tiles, whose records a second launch merges: 64 tokens over 2000 keys (32 / 8
+// heads) 87 -> 25 us, 1024 over 1024 (16 / 4) 89 -> 61, 256 over 512 (32 / 8) 37 ->
+// 23.  Fuller launches lose by the records' traffic (700 over 300, 32 / 8, 49
+// unsplit, 61 in two ranges; 2048 tokens 119, 173).
 // Of a served call: at least one token, so at least one block.
 Grid grid_of(const GqaShape &g, bool records)
 {
@@ -583,10 +582,9 @@ void launch_gqa_flash_split(hipStream_t stream, float *out, const float *query,
                             float *records)
 {
     const Grid d = grid_of(g, records != nullptr);
-    gqa_flash_split_kernel<<<d.token_tiles * d.ranges * g.key_value_heads, kThreads, 0,
+    gqa_flash_split_kernel<<<d.token_tiles * d.ranges * g.key_value_heads, kTeams * kThreads, 0,
                              stream>>>(out, query, key_cache, value_cache, g, d.tile_tokens,
-                                       d.token_tiles, d.token_tiles * g.key_value_heads <= kResident && d.ranges == 1,
-                             d.ranges, d.range_tiles, records);
+                                       d.token_tiles, d.ranges, d.range_tiles, records);
     if (d.ranges > 1) {
         const uint32_t pairs = uint32_t(g.tokens) * g.query_heads;
         gqa_flash_merge_kernel<<<(pairs + 3) / 4, 256, 0, stream>>>(out, records, d.ranges, pairs);

@@ -1,13 +1,12 @@
-"""The 64-wide prefill attention on split binary16 operands
+"""The 64-wide prefill attention on split bfloat16 operands
 (runtime_amd/csrc/gqa_flash.hip) at the edges of its tiles and key ranges, over
 the number range, and with infinities and NaN, against 64-bit softmax.
 
-Bound.  With s = sum_d |q_d k_d| / 8 of a (row, key) pair: halves drop at most
-3 * 2^-22 of each product, twelve f32 accumulations round by 2^-24 of at most s,
-and components below 2^-18 of a row's (tile's) largest carry 2^-40 of it, so a
-score is off by at most d = 2^-20 s + 2^-38 max|k| sum|q| / 8.  Probabilities
-then move by a factor within 2 d (both in the exponent and in the sum), plus
-2^-20 for exponent, halves and sums, and values by 2^-39 of the head's largest.
+Bound.  With s = sum_d |q_d k_d| / 8 of a (row, key) pair: the parts drop at most
+2 * 2^-24 of each product and twelve f32 accumulations round by 2^-24 of at most s
+each, so a score is off by at most d = 2^-20 s.  Probabilities then move by a
+factor within 2 d (both in the exponent and in the sum), plus 2^-20 for exponent,
+parts and sums.
 """
 from __future__ import annotations
 
@@ -33,11 +32,10 @@ def reference(q, k, v, start, qh, kvh):
         score = np.where(hidden, -np.inf, qq @ kk.T / 8.0)
         p = np.exp(score - score.max(axis=1, keepdims=True))
         p /= p.sum(axis=1, keepdims=True)
-        off = (2.0 ** -20 * (np.abs(qq) @ np.abs(kk).T) +
-               2.0 ** -38 * np.abs(kk).max() * np.abs(qq).sum(axis=1, keepdims=True)) / 8.0
+        off = 2.0 ** -20 * (np.abs(qq) @ np.abs(kk).T) / 8.0
         off = np.where(hidden, 0.0, off).max(axis=1, keepdims=True)
         want[:, h] = p @ vv
-        bound[:, h] = ((2 * off + 2.0 ** -20) * (p @ np.abs(vv)) + 2.0 ** -39 * np.abs(vv).max())
+        bound[:, h] = (2 * off + 2.0 ** -20) * (p @ np.abs(vv))
     return want.reshape(tokens, -1), bound.reshape(tokens, -1)
 
 
@@ -96,6 +94,48 @@ def test_number_range(backend, case):
     else:
         for a in (q, k, kc, v, vc):
             a[:] = 0
+    check(backend, q, k, v, kc, vc, start, qh, kvh)
+
+
+@pytest.mark.parametrize("start", [0, 100, 2000])
+@pytest.mark.parametrize("case", ["component", "elements", "later row", "large then small",
+                                  "2^-120", "2^100", "2^-105 among ones"])
+def test_values_of_very_different_size(backend, case, start):
+    """Every output keeps its own relative error, whatever stands beside its
+    operands in a tile."""
+    say("flash spread", case, start)
+    tokens, qh, kvh = 160, 16, 4
+    q, k, v, kc, vc = operands(9150 + start, tokens, start, qh, kvh)
+    rng = np.random.default_rng(9160 + start)
+    if case == "component":  # dimensions far below the largest
+        gain = np.exp2(-np.arange(D) / 2).astype(np.float32)
+        for a in (v, vc):
+            a *= np.tile(gain, kvh)
+    elif case == "elements":
+        for a in (v, vc):
+            a *= np.exp2(rng.uniform(-40, 40, a.shape)).astype(np.float32)
+        for a in (k, kc):
+            a *= np.exp2(rng.uniform(-40, 2, a.shape)).astype(np.float32)
+    elif case == "later row":  # a key that the rows before it must not see
+        v[70] *= np.float32(2.0 ** 45)
+        k[70] *= np.float32(2.0 ** 45)
+        q[70:] = 0  # (scores past 2^45 differ by more than any softmax resolves)
+    elif case == "large then small":
+        for a in (vc, v):
+            a[:max(start, 64) // 2] *= np.float32(2.0 ** 40)
+        q *= np.float32(4)
+    elif case == "2^-120":
+        v *= np.float32(2.0 ** -120)
+        vc *= np.float32(2.0 ** -120)
+    elif case == "2^100":
+        v *= np.float32(2.0 ** 100)
+        vc *= np.float32(2.0 ** 100)
+        k *= np.float32(2.0 ** 70)
+        kc *= np.float32(2.0 ** 70)
+        q *= np.float32(2.0 ** -70)
+    else:
+        v[::3] *= np.float32(2.0 ** -105)
+        k[::5] *= np.float32(2.0 ** -105)
     check(backend, q, k, v, kc, vc, start, qh, kvh)
 
 
