@@ -1574,16 +1574,20 @@ uint32_t gqa_splits(const GqaShape &g)
     return uint32_t(splits);
 }
 
-// The matrix-core prefill kernels serve heads of 16..kFlashMaxDim dimensions
-// in steps of 16, groups of at most kFlashRows query heads, and 16-byte aligned
-// operands (their float4 loads and stores).
+// The matrix-core prefill kernels serve 16-byte aligned operands (their float4
+// loads and stores), heads of 16..kFlashMaxDim dimensions in steps of 16 and groups
+// of at most kFlashRows query heads; head width 64 has a kernel, and limits, of its
+// own.
 bool flash_served(const GqaShape &g, const float *out, const float *query, const float *key_cache,
                   const float *value_cache)
 {
     auto aligned = [](const float *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    if (!aligned(out) || !aligned(query) || !aligned(key_cache) || !aligned(value_cache))
+        return false;
+    if (g.head_dim == 64)
+        return gqa_flash_split_served(g);
     return g.head_dim && g.head_dim % 16 == 0 && g.head_dim <= kFlashMaxDim && g.group >= 1 &&
-           g.group <= kFlashRows && (g.head_dim != 64 || gqa_flash_split_served(g)) && aligned(out) && aligned(query) && aligned(key_cache) &&
-           aligned(value_cache);
+           g.group <= kFlashRows;
 }
 
 template <int D>
@@ -1621,9 +1625,13 @@ size_t gqa_scratch_bytes(const GqaShape &g)
                   : 0;
 }
 
-size_t gqa_optional_scratch_bytes(const GqaShape &g)
+size_t gqa_optional_scratch_bytes(const GqaShape &g, const float *out, const float *query,
+                                  const float *key_cache, const float *value_cache)
 {
-    return !gqa_splits(g) && gqa_flash_split_served(g) ? gqa_flash_records_bytes(g) : 0;
+    return !gqa_splits(g) && g.head_dim == 64 &&
+                   flash_served(g, out, query, key_cache, value_cache)
+               ? gqa_flash_records_bytes(g)
+               : 0;
 }
 
 void launch_gqa(hipStream_t stream, float *out, const float *query, const float *key,

@@ -717,15 +717,21 @@ mfh_status mfh_causal_gqa(mfh_ctx *ctx, mfh_buf *output, const mfh_buf *query,
     g.head_dim = head_dim;
     g.group = query_heads / key_value_heads;
     g.scale = 1.0f / std::sqrt(float(head_dim));
-    float *partials = nullptr;
-    const size_t need = gqa_scratch_bytes(g);
-    if (const size_t bytes = need ? need : gqa_optional_scratch_bytes(g)) {
+    float *partials = nullptr, *records = nullptr;
+    size_t records_capacity = 0;
+    if (const size_t bytes = gqa_scratch_bytes(g)) {
         partials = static_cast<float *>(work_scratch(ctx, bytes));
-        if (!partials && need)
+        if (!partials)
             return allocation_failed(ctx);
+    } else if (const size_t useful =
+                   gqa_optional_scratch_bytes(g, dev_f32(output), dev_f32(query),
+                                              dev_f32(key_cache), dev_f32(value_cache))) {
+        partials = records =
+            static_cast<float *>(optional_block(ctx, useful, &records_capacity));
     }
     launch_gqa(ctx->stream, dev_f32(output), dev_f32(query), dev_f32(key), dev_f32(value),
                dev_f32(key_cache), dev_f32(value_cache), g, partials);
+    release_block(ctx, nullptr, records, records_capacity);
     if ((s = launched(ctx)))
         return s;
     *cache_len = new_len;

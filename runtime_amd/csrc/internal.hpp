@@ -222,6 +222,13 @@ mfh_status acquire_for(mfh_ctx *ctx, mfh_buf *owner, size_t bytes, void **out, s
 // Return a block (null is ignored); `owner` non-null uncharges its class.
 void release_block(mfh_ctx *ctx, mfh_buf *owner, void *ptr, size_t capacity);
 
+// A block for a call that runs faster with it and does without where it cannot have
+// one: an idle pool block, else a new one where the limit has room as things
+// stand, else null; nothing is evicted and no reason recorded.  The call returns it
+// (release_block) as soon as its kernels are queued, so it is idle, and makes room,
+// for the next allocation.
+void *optional_block(mfh_ctx *ctx, size_t bytes, size_t *capacity);
+
 // Device scratch owned by the context, grown on demand (stream ordered).
 // Null when the allocation is refused; acquire() recorded why, and
 // allocation_failed() is the status to return.

@@ -316,10 +316,11 @@ void launch_qk_norm_rope(hipStream_t stream, float *query_out, float *key_out, c
 // them at row `initial_len` of both caches), then attends.  Few (token,
 // head) pairs over long caches take a split-key path whose partials need
 // gqa_scratch_bytes(g) bytes of `scratch` (0: no scratch used).  Where that is
-// 0, gqa_optional_scratch_bytes(g) bytes may be given instead (0, or a null
-// `scratch`: none).
+// 0, a call with gqa_optional_scratch_bytes (0: it has no use for any) runs faster,
+// and without runs all the same.
 size_t gqa_scratch_bytes(const GqaShape &g);
-size_t gqa_optional_scratch_bytes(const GqaShape &g);
+size_t gqa_optional_scratch_bytes(const GqaShape &g, const float *out, const float *query,
+                                  const float *key_cache, const float *value_cache);
 void launch_gqa(hipStream_t stream, float *out, const float *query, const float *key,
                 const float *value, float *key_cache, float *value_cache, const GqaShape &g,
                 float *scratch);

@@ -411,10 +411,9 @@ mfh_status decode_step(mfl_model *m, const mfh_buf *device_ids, bool produce_log
                 g.group = da.group;
                 g.scale = da.scale;
                 float *partials = nullptr;
-                const size_t need = gqa_scratch_bytes(g);
-                if (const size_t bytes = need ? need : gqa_optional_scratch_bytes(g)) {
+                if (const size_t bytes = gqa_scratch_bytes(g)) {
                     partials = static_cast<float *>(work_scratch(c, bytes));
-                    if (!partials && need)
+                    if (!partials)
                         return allocation_failed(c);
                 }
                 launch_gqa(c->stream, dev(ws->attention), dev(ws->q_rope), nullptr, nullptr,

@@ -103,6 +103,14 @@ void evict(mfh_ctx *ctx)
     ctx->pool->evict_idle();
 }
 
+// Whether the limit has room for a new block of bucket(bytes).
+bool fits(const mfh_ctx *ctx, size_t bytes)
+{
+    const uint64_t want = pool_bucket(bytes);
+    const uint64_t owned = ctx->pool->reserved() + ctx->pending_result_bytes;
+    return owned + want >= owned && owned + want <= ctx->limits.max_total_bytes;
+}
+
 }  // namespace
 
 mfh_status acquire(mfh_ctx *ctx, size_t bytes, void **out, size_t *capacity)
@@ -112,15 +120,9 @@ mfh_status acquire(mfh_ctx *ctx, size_t bytes, void **out, size_t *capacity)
         return MFH_OK;
     // resources.rs:27-43 on the physical footprint: every pooled block, idle
     // ones included, plus pending readback staging.
-    const uint64_t want = pool_bucket(bytes);
-    const uint64_t limit = ctx->limits.max_total_bytes;
-    auto fits = [&] {
-        const uint64_t owned = ctx->pool->reserved() + ctx->pending_result_bytes;
-        return owned + want >= owned && owned + want <= limit;
-    };
-    if (!fits())
+    if (!fits(ctx, bytes))
         evict(ctx);
-    if (!fits())
+    if (!fits(ctx, bytes))
         return fail(ctx, MFH_RESOURCE_LIMIT, "allocation exceeds configured total resource limit");
     *out = ctx->pool->grow(bytes, capacity);
     if (!*out) {
@@ -131,6 +133,14 @@ mfh_status acquire(mfh_ctx *ctx, size_t bytes, void **out, size_t *capacity)
         return fail(ctx, MFH_RESOURCE_LIMIT, "device allocation failed");
     note_peak(ctx);
     return MFH_OK;
+}
+
+void *optional_block(mfh_ctx *ctx, size_t bytes, size_t *capacity)
+{
+    void *p = ctx->pool->take(bytes, capacity);
+    if (!p && fits(ctx, bytes) && (p = ctx->pool->grow(bytes, capacity)))
+        note_peak(ctx);
+    return p;
 }
 
 mfh_status acquire_for(mfh_ctx *ctx, mfh_buf *owner, size_t bytes, void **out, size_t *capacity)

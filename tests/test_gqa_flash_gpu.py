@@ -13,7 +13,9 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from tests.test_dense_gpu import rng_f32, run_gqa, say
+from runtime_amd.backend import CacheLength, GqaSpec, HipBackend, Limits
+from tests.test_dense_gpu import rng_f32, run_gqa, say, up
+from tests.test_resources_gpu import MIB, total
 
 pytestmark = pytest.mark.gpu
 D = 64
@@ -197,3 +199,37 @@ def test_no_tokens(backend, prefix, group):
     out, keys, values, length = run_gqa(backend, q, k, v, kc, vc, prefix, group, 1, D)
     assert out.shape == (0, group * D) and length == prefix
     assert np.array_equal(keys, kc) and np.array_equal(values, vc)
+
+
+@pytest.mark.parametrize("room", [24 * MIB, 2 * MIB])
+def test_key_ranges_leave_the_budget_alone(room):
+    """The key ranges' records (17 MB here) are memory the call does without:
+    with room for them, an allocation that takes that room afterwards succeeds;
+    without, the call runs, evicts no idle block and takes nothing."""
+    say("flash records", room)
+    tokens, start, qh, kvh = 1024, 1024, 16, 4
+    q, k, v, kc, vc = operands(9500, tokens, start, qh, kvh)
+    limit = 96 * MIB
+    be = HipBackend(0, limits=Limits(max_total_bytes=limit))
+    try:
+        bufs = [up(be, a) for a in (q, k, v, kc, vc)]
+        out = be.allocate_f32(q.shape)
+        idle = be.allocate_f32((MIB // 4,))
+        held = []
+        while (want := limit - total(be.resource_report()) - room) >= MIB:
+            held.append(be.allocate_f32(((1 << (want.bit_length() - 1)) // 4,)))
+        idle.release()
+        before = total(be.resource_report())
+        assert room <= limit - before < room + MIB
+        for _ in range(2):
+            be.causal_gqa(out, *bufs, CacheLength(start), GqaSpec(qh, kvh, D))
+            after = total(be.resource_report())
+            assert after > before if room > 17 * MIB else after == before
+        be.allocate_f32((1 << (room.bit_length() - 3),)).release()
+        for buf in held:  # room for the readback
+            buf.release()
+        want, bound = reference(q, np.concatenate([kc[:start], k]),
+                                np.concatenate([vc[:start], v]), start, qh, kvh)
+        assert np.all(np.abs(be.read(out).astype(np.float64) - want) <= bound)
+    finally:
+        be.close()
