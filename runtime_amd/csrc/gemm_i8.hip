@@ -489,7 +489,7 @@ bool gemm_i8_served(const PackedCall &call)
     const uint32_t columns = call.epilogue == Epilogue::Single ? 128 : 64;
     const uint64_t blocks =
         uint64_t((call.m + 31) / 32) * ((uint64_t(call.n) + columns - 1) / columns);
-    return call.format == Format::Int8 && !call.single_half &&
+    return call.format == Format::Int8 && !call.single_half && !call.halves &&
            (call.n < 4096 || blocks < 1024);
 }
 

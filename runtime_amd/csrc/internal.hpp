@@ -235,6 +235,9 @@ void *optional_block(mfh_ctx *ctx, size_t bytes, size_t *capacity);
 void *ids_scratch(mfh_ctx *ctx, size_t bytes);
 void *work_scratch(mfh_ctx *ctx, size_t bytes);
 void *digits_scratch(mfh_ctx *ctx, size_t bytes);
+// Whether digits_scratch(ctx, bytes) is within the limit as things stand (after a
+// refusal: with every idle block returned).  Allocates nothing.
+bool digits_scratch_fits(const mfh_ctx *ctx, size_t bytes);
 inline mfh_status allocation_failed(mfh_ctx *) { return MFH_RESOURCE_LIMIT; }
 
 // An F32 rank-2 buffer of binary16 file values: the 2-byte values are

@@ -99,6 +99,8 @@ struct PackedCall {
     bool separate_prologue = false;
     // Matrix-core GEMM: activations as one binary16 half instead of hi + lo.
     bool single_half = false;
+    // Matrix-core GEMM: the binary16-halves plan where a digit plan would serve.
+    bool halves = false;
     // Matrix-core GEMV only: a transform other than Plain replaces `x`.
     XForm xform;
     // Matrix-core GEMV, Single epilogue only: when non-zero, the launch

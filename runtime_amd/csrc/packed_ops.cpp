@@ -3,6 +3,7 @@
 // Admission restates CpuBackend's checks in the reference's order and with
 // its messages (crates/backend-cpu/src/packed.rs:11-466): every operand is
 // validated before anything is enqueued, so a rejected call writes nothing.
+#include <algorithm>
 #include <vector>
 
 #include "internal.hpp"
@@ -147,6 +148,37 @@ mfh_status prepare_streams(mfh_ctx *ctx, PackedCall *call, const mfh_buf *codes_
     return s;
 }
 
+// A ternary GEMM in `bytes` of scratch, fewer than it asks for: in the largest
+// pieces of 16, 32, 64, .. rows that fit, or else on the FP32 FMA kernel, which
+// needs none.
+void launch_ternary_pieces(hipStream_t stream, const PackedCall &call, void *scratch,
+                           size_t bytes)
+{
+    auto piece = [&](uint32_t first, uint32_t rows) {
+        PackedCall p = call;
+        p.m = std::min(rows, call.m - first);
+        p.x += size_t(first) * call.k;
+        p.out_a += size_t(first) * call.n;
+        if (p.out_b)
+            p.out_b += size_t(first) * call.n;
+        return p;
+    };
+    uint32_t rows = 16;
+    while (rows < call.m)
+        rows *= 2;
+    while ((rows /= 2) >= 16) {
+        // (A shorter last piece may split K further, and need more.)
+        const uint32_t last = (call.m - 1) / rows * rows;
+        if (gemm_mfma_scratch_bytes(piece(0, rows)) > bytes ||
+            gemm_mfma_scratch_bytes(piece(last, rows)) > bytes)
+            continue;
+        for (uint32_t first = 0; first < call.m; first += rows)
+            launch_gemm_mfma(stream, piece(first, rows), scratch);
+        return;
+    }
+    launch_gemm_fma(stream, call);
+}
+
 // Enqueue the kernels of one admitted packed product.  `a`/`b` are the
 // weight operands (b only for two-stream calls).
 mfh_status run_packed(mfh_ctx *ctx, PackedCall call, const mfh_buf *codes_a,
@@ -179,19 +211,23 @@ mfh_status run_packed(mfh_ctx *ctx, PackedCall call, const mfh_buf *codes_a,
             return s;
         call.single_half = ctx->gemm_activations == 1;
         void *scratch = digits_scratch(ctx, gemm_mfma_scratch_bytes(call));
+        // The digit records round the rows up to 16, so a budget that holds plain
+        // halves may refuse them: INT8 then runs on the halves, and ternary weights,
+        // which have no exact kernel on them, in pieces within as much memory
+        // (fewer than 16 rows take none of it).
+        const bool pieces = !scratch && gemm_mx_served(call);
         if (!scratch) {
-            // The digit records round the rows up to 16, so a budget that
-            // holds plain halves may refuse them: such a call still runs, on
-            // the FP32 FMA kernel, which needs no scratch.
-            if (!(gemm_mx_served(call) || gemm_i8_served(call)) ||
-                !digits_scratch(ctx, gemm_halves_scratch_bytes(call)))
+            call.halves = true;
+            const size_t bytes = gemm_halves_scratch_bytes(call);
+            if (pieces && call.m < 16 ? !digits_scratch_fits(ctx, bytes)
+                                      : !(scratch = digits_scratch(ctx, bytes)))
                 return allocation_failed(ctx);
-            launch_gemm_fma(stream, call);
-            return hipGetLastError() == hipSuccess
-                       ? MFH_OK
-                       : fail(ctx, MFH_BACKEND_FAILURE, "packed kernel launch failed");
         }
-        launch_gemm_mfma(stream, call, scratch);
+        if (pieces)
+            launch_ternary_pieces(stream, call, scratch,
+                                  scratch ? ctx->digits_scratch_capacity : 0);
+        else
+            launch_gemm_mfma(stream, call, scratch);
     } else {
         launch_gemm_fma(stream, call);
     }

@@ -244,12 +244,17 @@ void mark_written(mfh_buf *buf)
     }
 }
 
+static size_t scratch_size(size_t bytes)
+{
+    return bytes < (size_t(1) << 20) ? size_t(1) << 20 : bytes;
+}
+
 // Scratch blocks only grow; a replaced block returns to the pool, where
 // stream order keeps it from being reused before the work queued on it ran.
 static void *grow(mfh_ctx *ctx, void **slot, size_t *capacity, size_t bytes)
 {
     if (bytes > *capacity) {
-        size_t want = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
+        const size_t want = scratch_size(bytes);
         void *p = nullptr;
         size_t got = 0;
         if (acquire(ctx, want, &p, &got))
@@ -274,6 +279,11 @@ void *work_scratch(mfh_ctx *ctx, size_t bytes)
 void *digits_scratch(mfh_ctx *ctx, size_t bytes)
 {
     return grow(ctx, &ctx->digits_scratch, &ctx->digits_scratch_capacity, bytes);
+}
+
+bool digits_scratch_fits(const mfh_ctx *ctx, size_t bytes)
+{
+    return bytes <= ctx->digits_scratch_capacity || fits(ctx, scratch_size(bytes));
 }
 
 }  // namespace mfh

@@ -211,3 +211,44 @@ def test_scratch_limit(room, runs):
             assert np.array_equal(be.read(out), sentinel)
     finally:
         be.close()
+
+
+@pytest.mark.parametrize("m,n,room,runs", [(9, 64, MIB + 16384, True), (17, 16, 1400000, True),
+                                           (33, 16, 2700000, True), (33, 16, 2200000, False)])
+def test_scratch_limit_in_pieces(m, n, room, runs):
+    """A budget that holds the binary16-halves plan's scratch but not the digit
+    records of all rows: pieces of the rows run where their records fit (17 rows as
+    16 + 1, 33 as 32 + 1), and what does not (9 rows) takes no memory; less than
+    the halves plan's need refuses."""
+    say("mx scratch pieces", m, room)
+    k = 16384
+    codes, scales = make_weights(n, k, "ternary", 0x5EED0780)
+    x = convert.normal((m, k), 0xAC70780)
+    limit = 64 * MIB
+    be = HipBackend(0, limits=Limits(max_total_bytes=limit))
+    try:
+        cb, sb = upload_weights(be, codes, scales)
+        xb = be.upload_f32(x.shape, x)
+        out, out_b = be.allocate_f32((m, n)), be.allocate_f32((m, n))
+        be.prepare_packed(cb, sb)
+        fill = []
+        while (want := limit - total(be.resource_report()) - room) >= 1024:
+            size = 1 << (want.bit_length() - 1) if want > MIB else want // 256 * 256
+            fill.append(be.allocate_f32_classified((size // 4,), 1))
+        left = limit - total(be.resource_report())
+        assert room <= left < room + 1024
+        if not runs:
+            with pytest.raises(ExecutorError) as e:
+                be.packed_linear(out, xb, cb, sb)
+            assert e.value.variant == "ResourceLimit"
+            return
+        be.packed_linear(out, xb, cb, sb)
+        taken = left - (limit - total(be.resource_report()))
+        assert taken == 0 if m == 9 else 0 < taken <= room
+        check(be.read(out), x, codes, scales)
+        if m == 17:  # the pair's halves fit the same block
+            be.packed_linear_pair(out, out_b, xb, cb, sb, cb, sb)
+            assert np.array_equal(be.read(out), be.read(out_b))
+            check(be.read(out), x, codes, scales)
+    finally:
+        be.close()
