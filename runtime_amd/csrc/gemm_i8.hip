@@ -418,12 +418,17 @@ struct Plan {
 // that asked for 1000 took smaller tiles: M = 100 x 8192 x 2048 43 us against 29.5,
 // M = 300 x 4608 x 1024 30.4 against 23.8), and for a launch of one-tile waves still
 // short of blocks K runs of at least four groups.  us per call, before (two binary16
-// passes) -> now: M = 2048 x 2048 x 8192 185 -> 163, 1024 x 2048 x 2048 37.9 ->
-// 26.6, 128 x 2048 x 1024 15.0 -> 10.0, 16 x 8192 x 2048 16.5 -> 11.7; gate/up pairs
-// with SwiGLU M = 346 x 2560 x 1024 24.4 -> 18.4, 100 x 8192 x 2048 33.6 -> 29.5.
+// passes) -> now: M = 2048 x 2048 x 8192 184 -> 160, 1024 x 2048 x 2048 36.6 ->
+// 26.6, 128 x 2048 x 1024 15.0 -> 10.3, 16 x 8192 x 2048 16.5 -> 11.8; gate/up pairs
+// with SwiGLU M = 346 x 2560 x 1024 24.4 -> 19.1, 100 x 8192 x 2048 33.6 -> 29.5.
 // Four column tiles per wave (two waves per SIMD instead of four) took 344 against
 // 324 us on the pair M = 2048 x 8192 x 2048.  Error against 64-bit sums 5.3e-7 ->
 // 2.7e-7 (2048 x 8192 x 2048).
+//
+// Weights of 2^24 values and more are read once per 16 TI rows from beyond the L2s:
+// there 100 blocks are enough (M = 128 x 8192 x 8192 82 us with small tiles, 53 with
+// large ones, 57 on the halves; 64 x 8192 x 4096 30, 23, 25; pairs 128 x 4096 x 4096
+// 46, 32, 34; the other way only 48 x 16384 x 2048 21, 23, 24).
 Plan plan_of(const PackedCall &call)
 {
     const uint32_t s = call.epilogue == Epilogue::Single ? 1 : 2;
@@ -434,7 +439,7 @@ Plan plan_of(const PackedCall &call)
         p.tiles = p.tiles_n * ((row_tiles + ti - 1) / ti);
         return p;
     };
-    constexpr uint32_t enough = 400;
+    const uint32_t enough = uint64_t(call.n) * call.k * s >= 1u << 24 ? 100 : 400;
     Plan p = with(2, 2);
     if (p.tiles < enough)
         p = with(1, 2);
@@ -481,9 +486,13 @@ size_t records_bytes(const PackedCall &call)
 }  // namespace
 
 // The binary16-halves kernel keeps the launches that fill the device with its
-// 64-row tiles over wide outputs: M = 512 x 8192 x 2048 46.5 us there, 48.9 here, M
-// = 2048 x 8192 x 2048 177 both, against 58 and 46 at M = 2048 x 2048 x 2048 (as
-// many blocks, fewer columns) and 185 and 163 at M = 2048 x 2048 x 8192.
+// 64-row tiles over wide outputs, where both take the same time within 5 % (us,
+// halves and here: M = 1024 x 8192 x 2048 86.8, 89.9; 2048 x 8192 x 2048 171, 173;
+// 2048 x 4096 x 8192 334, 337; 512 x 8192 x 2048 50.0, 48.0; at its edge 1024 x 4096
+// x 2048 48.0, 43.6).  Outside, here is faster: 2048 x 2048 x 2048 51.7, 44.7 (as many
+// blocks, fewer columns), 2048 x 2048 x 8192 184, 160, 512 x 4096 x 8192 98, 89, 256
+// x 6144 x 2048 31.9, 25.8, 128 x 4096 x 2048 24.8, 17.5; K = 8192 at 48-96 rows is the
+// closest (96 x 4096 x 8192 32.7, 34.3).
 bool gemm_i8_served(const PackedCall &call)
 {
     const uint32_t columns = call.epilogue == Epilogue::Single ? 128 : 64;
