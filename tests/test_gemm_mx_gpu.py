@@ -40,8 +40,8 @@ def check(got, x, codes, scales, floor=0.0):
 
 # One to two row tiles around 16 and 32 rows, column tiles around 64, 128 and
 # 256, one group, K runs that start inside a 256-wide tile load (3456 and 2816
-# split into runs of 9 and 11 groups), and launches of every wave tile:
-# 1 x 1, 1 x 2 (long K), 2 x 2, 2 x 4.
+# split into runs of 9 and 11 groups), and launches of 1 x 1, 2 x 2 and 2 x 4 wave
+# tiles (1 x 2: test_wave_tiles).
 SHAPES = [(9, 16, 128), (15, 63, 256), (16, 65, 384), (17, 129, 640), (31, 257, 1280),
           (33, 1000, 3456), (20, 70, 2816), (48, 512, 8192), (200, 1100, 4096), (130, 4608, 1024),
           (400, 4100, 256), (1025, 3300, 128), (2048, 2049, 384)]
@@ -53,6 +53,30 @@ def test_edges(backend, m, n, k):
     codes, scales = make_weights(n, k, "ternary", 0x5EED0700 + n + k)
     x = convert.normal((m, k), 0xAC70700 + m)
     check(run_linear(backend, x, codes, scales), x, codes, scales)
+
+
+# (rows, columns, width, streams): 1 x 2 wave tiles (enough blocks, long K) and a
+# pair's 2 x 2 and 2 x 4 ones.
+TILES = [(330, 2500, 256, 1), (300, 1300, 4096, 1), (1030, 2050, 256, 2), (1030, 4100, 384, 2)]
+
+
+@pytest.mark.parametrize("m,n,k,streams", TILES)
+def test_wave_tiles(backend, m, n, k, streams):
+    say("mx wave tiles", m, n, k, streams)
+    weights = [make_weights(n, k, "ternary", 0x5EED07A0 + n + k + i) for i in range(streams)]
+    x = convert.normal((m, k), 0xAC70800 + m)
+    if streams == 1:
+        check(run_linear(backend, x, *weights[0]), x, *weights[0])
+        return
+    bufs = [upload_weights(backend, *w) for w in weights]
+    xb = backend.upload_f32(x.shape, x)
+    outs = [backend.allocate_f32((m, n)) for _ in range(3)]
+    backend.packed_linear_pair(*outs[:2], xb, *bufs[0], *bufs[1])
+    backend.packed_swiglu_pair(outs[2], xb, *bufs[0], *bufs[1])
+    a, b, fused = (backend.read(out) for out in outs)
+    check(a, x, *weights[0])
+    check(b, x, *weights[1])
+    np.testing.assert_allclose(fused, oracle.swiglu(a, b), rtol=2e-6, atol=1e-30)
 
 
 @pytest.mark.parametrize("m,n,k", [(9, 40, 384), (70, 300, 1024), (300, 2600, 256)])
