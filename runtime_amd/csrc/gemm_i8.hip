@@ -328,53 +328,62 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_i8_kernel(I8Args g)
         }
     if (__builtin_expect(__any(nan != nan || odd_scale), 0)) {
         // A tile at a time, straight from memory.
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int jt = 0; jt < TJ; ++jt) {
-                if (mt0 + i >= g.row_tiles)
-                    continue;
-                v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-                for (uint32_t gr = g_begin; gr < g_end; ++gr) {
-                    const uint8_t *rec = x_src + gr * x_step + i * kRecord;
-                    const char *w = wptr[jt] + size_t(gr) * 2048 + 16 * lane;
-                    const char *sp = sptr[jt] + (size_t(gr) * 16 + li) * sizeof(Scale);
-                    float gs;
-                    if constexpr (HALF)
-                        gs = __half2float(*reinterpret_cast<const __half *>(sp));
-                    else
-                        gs = *reinterpret_cast<const float *>(sp);
-                    int gs_exp = 0;
-                    const float gs_frac = frexpf(gs, &gs_exp);
-                    v4i digit[kDigits];
+        for (uint32_t tile = 0; tile < uint32_t(TI * TJ); ++tile) {
+            if (mt0 + tile / TJ >= g.row_tiles)
+                break;
+            const uint32_t st = tile % TJ / TJS, t = n0 / 16 + wave * TJS + tile % TJS;
+            const size_t live = t < g.n_tiles ? t : 0;
+            const char *const w_tile =
+                reinterpret_cast<const char *>(g.wtiles[st]) + live * g.tile_vecs * 16;
+            const char *const s_tile = static_cast<const char *>(g.scales[st]) +
+                                       live * g.groups_pad * 16 * (HALF ? 2 : 4);
+            v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+            for (uint32_t gr = g_begin; gr < g_end; ++gr) {
+                const uint8_t *rec = x_src + gr * x_step + tile / TJ * kRecord;
+                const char *w = w_tile + size_t(gr) * 2048 + 16 * lane;
+                const char *sp = s_tile + (size_t(gr) * 16 + li) * sizeof(Scale);
+                float gs;
+                if constexpr (HALF)
+                    gs = __half2float(*reinterpret_cast<const __half *>(sp));
+                else
+                    gs = *reinterpret_cast<const float *>(sp);
+                int gs_exp = 0;
+                const float gs_frac = frexpf(gs, &gs_exp);
+                v4i digit[kDigits];
 #pragma unroll
-                    for (int d = 0; d < kDigits; ++d) {
-                        digit[d] = v4i{0, 0, 0, 0};
+                for (int d = 0; d < kDigits; ++d) {
+                    digit[d] = v4i{0, 0, 0, 0};
 #pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            digit[d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-                                *reinterpret_cast<const v4i *>(rec + d * kDigitBytes + 1024 * h +
-                                                               16 * lane),
-                                *reinterpret_cast<const v4i *>(w + 1024 * h), digit[d], 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float whole = fmaf(float((digit[0][r] << 8) + digit[1][r]), 256.0f,
-                                                 float(digit[2][r]));
-                        const uint32_t unit =
-                            reinterpret_cast<const uint32_t *>(rec + kUnitsAt)[4 * lq + r];
-                        int exp = 0;
-                        float frac = frexpf(__uint_as_float(unit), &exp);
-                        if (is_code(unit)) {
-                            exp = int((unit >> 13) & 511) - kCodeBias;
-                            frac = __uint_as_float(0x3f800000u | (unit & 0x1fffu) << 10);
-                        }
-                        sum[r] += ldexpf(whole * (frac * gs_frac), exp + gs_exp);
-                    }
+                    for (int h = 0; h < 2; ++h)
+                        digit[d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                            *reinterpret_cast<const v4i *>(rec + d * kDigitBytes + 1024 * h +
+                                                           16 * lane),
+                            *reinterpret_cast<const v4i *>(w + 1024 * h), digit[d], 0, 0, 0);
                 }
-                total[i][jt] = sum;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float whole = fmaf(float((digit[0][r] << 8) + digit[1][r]), 256.0f,
+                                             float(digit[2][r]));
+                    const uint32_t unit =
+                        reinterpret_cast<const uint32_t *>(rec + kUnitsAt)[4 * lq + r];
+                    int exp = 0;
+                    float frac = frexpf(__uint_as_float(unit), &exp);
+                    if (is_code(unit)) {
+                        exp = int((unit >> 13) & 511) - kCodeBias;
+                        frac = __uint_as_float(0x3f800000u | (unit & 0x1fffu) << 10);
+                    }
+                    sum[r] += ldexpf(whole * (frac * gs_frac), exp + gs_exp);
+                }
             }
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int jt = 0; jt < TJ; ++jt)
+                    if (tile == uint32_t(i * TJ + jt))
+                        total[i][jt] = sum;
+        }
     }
 
 #pragma unroll

@@ -395,60 +395,69 @@ __global__ __launch_bounds__(kThreads, 3) void gemm_mx_kernel(MxArgs g)
     if (__builtin_expect(__any(nan != nan), 0)) {
         // A tile at a time, straight from memory, on signed levels.
         const uint32_t at = cold_lane(), ci = at & 15, cq = at >> 4;
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int jt = 0; jt < TJ; ++jt) {
-                if (mt0 + i >= g.row_tiles)
-                    continue;
-                v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-                for (uint32_t gr = g_begin; gr < g_end; ++gr) {
-                    const uint8_t *rec = x_src + gr * x_step + i * kRecord;
-                    const v2u codes = *reinterpret_cast<const v2u *>(
-                        wptr[jt] + size_t(gr / 2) * 1024 + 16 * at + 8 * (gr & 1));
-                    v8i level = {};
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const unsigned w = ((codes[t / 2] ^ 0x80808080u) >> (2 * (t & 1))) &
-                                           0x33333333u;
-                        // Nibbles 0..3 to the FP4 values -0.5, 0, 0.5 and 1.
-                        const unsigned zero = ~(w | w >> 1) & 0x11111111u;
-                        level[t] = int((w - (zero ^ 0x11111111u)) | zero * 9);
-                    }
-                    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t tile = 0; tile < uint32_t(TI * TJ); ++tile) {
+            if (mt0 + tile / TJ >= g.row_tiles)
+                break;
+            const uint32_t st = tile % TJ / TJS, t = n0 / 16 + wave * TJS + tile % TJS;
+            const size_t live = t < g.n_tiles ? t : 0;
+            const char *const w_tile =
+                reinterpret_cast<const char *>(g.wtiles[st]) + live * g.tile_vecs * 16;
+            const char *const s_tile = static_cast<const char *>(g.scales[st]) +
+                                       live * g.groups_pad * 16 * (HALF ? 2 : 4);
+            v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-                    for (int d = kDigits - 1; d >= 0; --d) {
-                        const v4u lo =
-                            *reinterpret_cast<const v4u *>(rec + d * kDigitBytes + 16 * at);
-                        const v2u hi = *reinterpret_cast<const v2u *>(rec + d * kDigitBytes +
-                                                                      1024 + 8 * at);
-                        const v8i ad = {int(lo[0]), int(lo[1]), int(lo[2]), int(lo[3]),
-                                        int(hi[0]), int(hi[1]), 0, 0};
-                        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                            ad, level, acc, 2, 4, 0, int(rec[kExpsAt + at]), 0,
-                            128 - kDigitBits * d);
-                    }
-                    const char *sp = sptr[jt] + (size_t(gr) * 16 + ci) * sizeof(Scale);
-                    float gs;
-                    if constexpr (HALF)
-                        gs = __half2float(*reinterpret_cast<const __half *>(sp));
-                    else
-                        gs = *reinterpret_cast<const float *>(sp);
-                    int gs_exp = 0;
-                    const float gs_frac = frexpf(gs, &gs_exp);
+            for (uint32_t gr = g_begin; gr < g_end; ++gr) {
+                const uint8_t *rec = x_src + gr * x_step + tile / TJ * kRecord;
+                const v2u codes = *reinterpret_cast<const v2u *>(
+                    w_tile + size_t(gr / 2) * 1024 + 16 * at + 8 * (gr & 1));
+                v8i level = {};
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const uint32_t start =
-                            reinterpret_cast<const uint32_t *>(rec + kSumsAt)[4 * cq + r];
-                        if (start == kNanBits)
-                            sum[r] = nan_of(0);
-                        const int back = start == (kNanBits | kShifted) ? kShift : 0;
-                        sum[r] += ldexpf(acc[r] * gs_frac, gs_exp + back);
-                    }
+                for (int t = 0; t < 4; ++t) {
+                    const unsigned w = ((codes[t / 2] ^ 0x80808080u) >> (2 * (t & 1))) &
+                                       0x33333333u;
+                    // Nibbles 0..3 to the FP4 values -0.5, 0, 0.5 and 1.
+                    const unsigned zero = ~(w | w >> 1) & 0x11111111u;
+                    level[t] = int((w - (zero ^ 0x11111111u)) | zero * 9);
                 }
-                total[i][jt] = sum;
+                v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                for (int d = kDigits - 1; d >= 0; --d) {
+                    const v4u lo =
+                        *reinterpret_cast<const v4u *>(rec + d * kDigitBytes + 16 * at);
+                    const v2u hi = *reinterpret_cast<const v2u *>(rec + d * kDigitBytes +
+                                                                  1024 + 8 * at);
+                    const v8i ad = {int(lo[0]), int(lo[1]), int(lo[2]), int(lo[3]),
+                                    int(hi[0]), int(hi[1]), 0, 0};
+                    acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                        ad, level, acc, 2, 4, 0, int(rec[kExpsAt + at]), 0,
+                        128 - kDigitBits * d);
+                }
+                const char *sp = s_tile + (size_t(gr) * 16 + ci) * sizeof(Scale);
+                float gs;
+                if constexpr (HALF)
+                    gs = __half2float(*reinterpret_cast<const __half *>(sp));
+                else
+                    gs = *reinterpret_cast<const float *>(sp);
+                int gs_exp = 0;
+                const float gs_frac = frexpf(gs, &gs_exp);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t start =
+                        reinterpret_cast<const uint32_t *>(rec + kSumsAt)[4 * cq + r];
+                    if (start == kNanBits)
+                        sum[r] = nan_of(0);
+                    const int back = start == (kNanBits | kShifted) ? kShift : 0;
+                    sum[r] += ldexpf(acc[r] * gs_frac, gs_exp + back);
+                }
             }
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int jt = 0; jt < TJ; ++jt)
+                    if (tile == uint32_t(i * TJ + jt))
+                        total[i][jt] = sum;
+        }
     }
 
 #pragma unroll
