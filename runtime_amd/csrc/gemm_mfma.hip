@@ -1,6 +1,6 @@
-// Matrix-core prefill GEMM for packed NF4 weights, for INT8 ones where gemm_i8.hip
-// does not serve the call, and for ternary ones in single-half mode (m > 8; exact
-// ternary: gemm_mx.hip).
+// Matrix-core prefill GEMM (m > 8) for packed NF4 weights, for INT8 ones where
+// gemm_i8.hip does not serve the call or its scratch was refused, and for ternary
+// ones in single-half mode (exact ternary: gemm_mx.hip).
 //
 // out[m, n] = sum_g scale[n, g] * sum_{k in g} x[m, k] * level(code[n, k]),
 // the reference's group-then-scale order (kernels-simd/src/lib.rs:54,205).
@@ -242,8 +242,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
     // Waves along n (M = 2048 x 8192 x 2048 against 2 x 2: NF4 exact 218 ->
     // 206 us, INT8 exact 172 -> 165, single-half 3-9 % faster).
     constexpr int WN = 4;
-    constexpr int WM = 4 / WN;
-    constexpr int TI = BM / 16 / WM;             // 16-row MFMA tiles per wave
+    constexpr int TI = BM / 16;                  // 16-row MFMA tiles per wave
     constexpr int TJ = kBN / 16 / WN;            // 16-column MFMA tiles per wave
     constexpr int TJS = TJ / S;                  // column tiles per stream per wave
     constexpr int BNS = kBN / S;                 // block columns per stream
@@ -274,7 +273,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
     const int tid = threadIdx.x, lane = tid & 63;
     // Wave-uniform, so the tile addresses live in scalar registers.
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
     const int li = lane & 15, lq = lane >> 4;
     const uint32_t chunk_stages = g.k / kBK / g.chunks;
     const uint32_t s_begin = chunk * chunk_stages, s_end = s_begin + chunk_stages;
@@ -313,7 +311,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
 #pragma unroll
     for (int jt = 0; jt < TJ; ++jt) {
         const int st = jt / TJS, tt = jt % TJS;
-        const uint32_t t = n0 / 16 + wn * TJS + tt;
+        const uint32_t t = n0 / 16 + wave * TJS + tt;
         wlive[jt] = t < g.n_tiles;
         wptr[jt] = reinterpret_cast<const v4u *>(g.wtiles[st]) +
                    size_t(wlive[jt] ? t : 0) * g.tile_vecs + lane;
@@ -405,7 +403,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
             const int koff = F == Format::Nf4 ? 32 * h + 8 * lq : 16 * lq + 8 * h;
 #pragma unroll
             for (int i = 0; i < TI; ++i) {
-                const int row = wm * (BM / WM) + i * 16 + li;
+                const int row = i * 16 + li;
                 const v8h ah = *reinterpret_cast<const v8h *>(&As[buf][0][row][koff]);
                 const v8h al = *reinterpret_cast<const v8h *>(&As[buf][PA - 1][row][koff]);
 #pragma unroll
@@ -465,19 +463,19 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs g)
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const uint32_t mm = m0 + wm * (BM / WM) + i * 16 + lq * 4 + r;
+            const uint32_t mm = m0 + i * 16 + lq * 4 + r;
             rowf[i][r] = g.factor[mm < g.m ? mm : 0];
         }
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const uint32_t mm = m0 + wm * (BM / WM) + i * 16 + lq * 4 + r;
+            const uint32_t mm = m0 + i * 16 + lq * 4 + r;
             if (mm >= g.m)
                 continue;
 #pragma unroll
             for (int tt = 0; tt < TJS; ++tt) {
-                const uint32_t nn = n0 + (wn * TJS + tt) * 16 + li;
+                const uint32_t nn = n0 + (wave * TJS + tt) * 16 + li;
                 if (nn >= g.n)
                     continue;
                 const size_t o = size_t(mm) * g.n + nn;
@@ -605,15 +603,12 @@ uint32_t tiles_of(const PackedCall &call, uint32_t *tiles_n, uint32_t bm)
 // Rows per block tile: 64 where 128-row tiles would not fill the grid
 // without a K split (fewer than kHalfRowsBelow tiles), so the product
 // needs fewer K chunks (none at M = 512 x 8192) and their reduction --
-// except for ternary and NF4 at long K past 512 rows, where the 128-row
-// tiles and their split measured faster.  Measured (us per call, A/B on one device): M = 512 x
-// 8192 x 2048 ternary 58.4 -> 50.0, INT8 61.3 -> 50.0-50.9, NF4 70-73 ->
-// 62.6-63.5; M = 2048 x 2048 x 2048 ternary 63.5 -> 58.3-59.2, NF4 76.3 ->
-// 69.6; M = 128 35.6 -> 30.1; M = 256 41.8 -> 39.0; M = 512 x 2048 x 8192
-// 2-7 % faster; but M = 2048 x 2048 x 8192 ternary 156.1-156.6 with the
-// split against 159.8-160.1, NF4 209.2-209.5 against 213.5-214.5, M = 1024
-// ternary 95.8 against 98.7-100 (INT8 164.8-166.5 against 169.3-169.8: it
-// keeps the 64-row tiles).
+// except for single-half ternary and NF4 at long K past 512 rows, where the
+// 128-row tiles and their split measured faster.  Measured (us per call, 128-row ->
+// 64-row tiles, A/B on one device): M = 512 x 8192 x 2048 INT8 61.3 -> 50.0-50.9, NF4
+// 70-73 -> 62.6-63.5; M = 2048 x 2048 x 2048 NF4 76.3 -> 69.6; M = 512 x 2048 x
+// 8192 2-7 % faster; but M = 2048 x 2048 x 8192 NF4 209.2-209.5 with the split
+// against 213.5-214.5 (INT8 166.0 against 169.5: it keeps the 64-row tiles).
 constexpr uint32_t kHalfRowsBelow = 512;
 uint32_t block_rows(const PackedCall &call)
 {

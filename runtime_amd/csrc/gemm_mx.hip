@@ -17,7 +17,8 @@
 //   minus the row's sum over the group.
 // - v_mfma_scale_f32_16x16x128_f8f6f4 multiplies exactly, applies both block
 //   scales and accumulates in f32; a 128-group is five of them, the largest
-//   digit first, which cancels the start value at once.  The epilogue adds group_sum * scale in f32 (one FMA).
+//   digit first, which cancels the start value at once.  The epilogue adds
+//   group_sum * scale in f32 (one FMA).
 // - A row with a non-finite value gets NaN start values, so all of its
 //   outputs are NaN, as with a NaN or infinity in every dot.
 // - These are sums of true magnitudes (small ones keep their precision: the
@@ -500,12 +501,12 @@ struct Plan {
 // The largest wave tile that still gives the launch enough blocks: larger
 // tiles read each operand for more products, more blocks hide each other's
 // loads.  Enough is 400 blocks for a single product and 1000 for a pair
-// (us per call, larger / smaller tile: M = 2048 x 8192 x 2048 103 (2 x 4) /
-// 110 (2 x 2); M = 256 x 8192 x 2048 24.4 (256 blocks) / 22.0 (512); M = 346
-// x 2560 x 1024 13.1 (220) / 11.3 (440); M = 128 x 4608 x 1024 pair 13.5
-// (576) / 12.0 (1152)).  Four row tiles per wave (two waves per SIMD instead
-// of three) measured 109 us on the first shape and 136 against 110 on M = 2048
-// x 2048 x 8192.
+// (us per call, larger / smaller tile: M = 2048 x 8192 x 2048 109-114 (2 x 4)
+// / 127 (2 x 2), 2048 x 2048 x 8192 120-127 / 131; M = 256 x 8192 x 2048 24.4 (256
+// blocks) / 22.0 (512); M = 346 x 2560 x 1024 13.1 (220) / 11.3 (440); M = 128 x
+// 4608 x 1024 pair 13.5 (576) / 12.0 (1152)).  Four row tiles per wave (two waves
+// per SIMD instead of three), tried before the loop took two groups per iteration,
+// measured 109 against 103 us on the first shape and 136 against 110 on the second.
 //
 // A launch of one-tile waves that is still short of blocks splits K into runs
 // of at least four groups, up to 512 blocks, where that saves eight groups

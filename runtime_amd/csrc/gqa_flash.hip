@@ -539,7 +539,7 @@ constexpr uint32_t kResident = 256;
 
 // A launch that leaves half of the CUs idle cuts its keys into ranges of at least
 // four tiles, whose records a second launch merges: 64 tokens over 2000 keys (32 / 8
-// heads) 87 -> 25 us, 1024 over 1024 (16 / 4) 89 -> 61, 256 over 512 (32 / 8) 37 ->
+// heads) 87 -> 26 us, 1024 over 1024 (16 / 4) 89 -> 63, 256 over 512 (32 / 8) 37 ->
 // 23.  Fuller launches lose by the records' traffic (700 over 300, 32 / 8, 49
 // unsplit, 61 in two ranges; 2048 tokens 119, 173).
 // Of a served call: at least one token, so at least one block.
