@@ -226,7 +226,8 @@ void release_block(mfh_ctx *ctx, mfh_buf *owner, void *ptr, size_t capacity);
 // one: an idle pool block, else a new one where the limit has room as things
 // stand, else null; nothing is evicted and no reason recorded.  The call returns it
 // (release_block) as soon as its kernels are queued, so it is idle, and makes room,
-// for the next allocation.
+// for the next allocation.  Null under stream capture: the block would be another
+// buffer's by the time the graph runs.
 void *optional_block(mfh_ctx *ctx, size_t bytes, size_t *capacity);
 
 // Device scratch owned by the context, grown on demand (stream ordered).

@@ -137,6 +137,12 @@ mfh_status acquire(mfh_ctx *ctx, size_t bytes, void **out, size_t *capacity)
 
 void *optional_block(mfh_ctx *ctx, size_t bytes, size_t *capacity)
 {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess ||
+        capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     void *p = ctx->pool->take(bytes, capacity);
     if (!p && fits(ctx, bytes) && (p = ctx->pool->grow(bytes, capacity)))
         note_peak(ctx);

@@ -10,9 +10,12 @@ parts and sums.
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
+from runtime_amd import hiptime
 from runtime_amd.backend import CacheLength, GqaSpec, HipBackend, Limits
 from tests.test_dense_gpu import rng_f32, run_gqa, say, up
 from tests.test_resources_gpu import MIB, total
@@ -233,3 +236,40 @@ def test_key_ranges_leave_the_budget_alone(room):
         assert np.all(np.abs(be.read(out).astype(np.float64) - want) <= bound)
     finally:
         be.close()
+
+
+def test_capture_keeps_no_pool_block(backend):
+    """A captured call writes nothing but its output and caches when the graph
+    runs, whatever the pool's idle blocks hold by then."""
+    say("flash capture")
+    tokens, start, qh, kvh = 1024, 1024, 16, 4
+    q, k, v, kc, vc = operands(9600, tokens, start, qh, kvh)
+    want, bound = reference(q, np.concatenate([kc[:start], k]), np.concatenate([vc[:start], v]),
+                            start, qh, kvh)
+    bufs, out = [up(backend, a) for a in (q, k, v, kc, vc)], backend.allocate_f32(q.shape)
+    zeros = up(backend, np.zeros_like(q))
+
+    def call():
+        backend.causal_gqa(out, *bufs, CacheLength(start), GqaSpec(qh, kvh, D))
+
+    call()  # leaves its records' block idle
+    backend.synchronize()
+    hip, stream = hiptime.hip(), ctypes.c_void_p(backend.stream())
+    graph, program = ctypes.c_void_p(), ctypes.c_void_p()
+    hiptime.check(hip.hipStreamBeginCapture(stream, 0), "begin capture")
+    try:
+        call()
+    finally:
+        hiptime.check(hip.hipStreamEndCapture(stream, ctypes.byref(graph)), "end capture")
+    hiptime.check(hip.hipGraphInstantiate(ctypes.byref(program), graph, None, None,
+                                          ctypes.c_size_t(0)), "instantiate")
+    sentinel = np.full((tokens * qh * 2 * (D + 2),), 7.0, np.float32)  # takes that block
+    other = up(backend, sentinel)
+    for _ in range(3):
+        backend.copy(out, zeros)
+        hiptime.check(hip.hipGraphLaunch(program, stream), "launch")
+        backend.synchronize()
+        assert np.all(np.abs(backend.read(out).astype(np.float64) - want) <= bound)
+        assert np.array_equal(backend.read(other), sentinel)
+    hiptime.check(hip.hipGraphExecDestroy(program), "destroy")
+    hiptime.check(hip.hipGraphDestroy(graph), "destroy")
