@@ -4,9 +4,9 @@
 // Flash-style causal GQA for many (token, query head) pairs.  A block serves one
 // key/value head and kRows query rows: `tile_tokens` consecutive tokens times the
 // group's query heads (row r is token t0 + r / group, query head r % group of the
-// key/value head).  Its two teams of kWaves waves, 16 rows each, take the kKeys-key
-// tiles in turn, each through LDS tiles of its own that every row of the team
-// shares, and the first team adds the second's rows to its own in the end.
+// key/value head).  Its one or two teams of kWaves waves, 16 rows each, take the
+// kKeys-key tiles in turn, each through LDS tiles of its own that every row of the
+// team shares, and the first team adds the second's rows to its own in the end.
 //
 // Exactness plan.  Every query, key, value and probability is the sum of three
 // bfloat16 parts that hold all 24 bits (bfloat16 has the exponents of f32, so no
@@ -34,7 +34,7 @@
 //
 // Bound.  Per wave and tile 96 MFMAs (1536 cycles) and about 350 vector
 // instructions (1400 cycles) of softmax and splitting, which hardly overlap: they
-// take 80 % of the time.  2048 tokens, 32 / 8 heads: 119 us per call with the cache
+// take 80 % of the time.  2048 tokens, 32 / 8 heads: 117 us per call with the cache
 // append, 227 on the fp32 matrix cores (128 MFMAs of 32 cycles per tile), 100 on
 // binary16 hi + lo halves with shared scales, which lost small values beside large
 // ones; error against 64-bit sums 1.8e-7 (fp32 matrix cores 4.0e-7, halves 2.6e-7;
@@ -57,7 +57,6 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
-constexpr int kTeams = 2;
 constexpr int kWaves = 8;  // per team, of 16 rows each
 constexpr uint32_t kThreads = 64 * kWaves;  // per team
 constexpr uint32_t kRows = 16 * kWaves;
@@ -162,7 +161,8 @@ __device__ __forceinline__ v4f multiply_add(const Parts &a, const Parts &b, v4f 
     return multiply_add(a.hi, b.hi, c);
 }
 
-__global__ __launch_bounds__(kTeams * kThreads, 4) void gqa_flash_split_kernel(
+template <int TEAMS>
+__global__ __launch_bounds__(TEAMS * kThreads, 4) void gqa_flash_split_kernel(
     float *__restrict__ out, const float *__restrict__ query, const float *__restrict__ key_cache,
     const float *__restrict__ value_cache, GqaShape g, uint32_t tile_tokens, uint32_t token_tiles,
     uint32_t ranges, uint32_t range_tiles, float *__restrict__ records)
@@ -170,9 +170,12 @@ __global__ __launch_bounds__(kTeams * kThreads, 4) void gqa_flash_split_kernel(
     // Per team the parts of a key tile and of a transposed value tile; in the end
     // the second team's accumulators.
     constexpr uint32_t kTile = kParts * kPlane;
-    __shared__ __align__(1024) uint8_t lds[kTeams][2 * kTile];
+    __shared__ __align__(1024) uint8_t lds[TEAMS][2 * kTile];
     // The parts of the rows' queries, [part][step].
     __shared__ __align__(1024) v4u q_lds[kParts][2][kThreads];
+    __shared__ uint32_t any_bad;
+    if (threadIdx.x == 0)
+        any_bad = 0;
 
     const uint32_t tid = threadIdx.x % kThreads, lane = tid & 63;
     const uint32_t team = __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads);
@@ -316,8 +319,8 @@ __global__ __launch_bounds__(kTeams * kThreads, 4) void gqa_flash_split_kernel(
     // the tile's keys are complete and the values of the tile before are free, behind
     // the second the tile's values are complete and its keys are free.  The values
     // (the next keys) to store there were requested half a tile earlier.
-    for (uint32_t first = begin; first < end; first += kTeams) {
-        const uint32_t n = first + team, next = n + kTeams;
+    for (uint32_t first = begin; first < end; first += TEAMS) {
+        const uint32_t n = first + team, next = n + TEAMS;
         const uint32_t k0 = n * kKeys;
         const bool active = n < end && k0 <= wave_last && !q_bad;
         __syncthreads();
@@ -406,14 +409,16 @@ __global__ __launch_bounds__(kTeams * kThreads, 4) void gqa_flash_split_kernel(
             }
         }
     }
-    // (A barrier, so the tiles are free.)
-    if (__syncthreads_or(bad) || q_bad) {
+    if (bad)
+        any_bad = 1;
+    __syncthreads();  // and the tiles are free
+    if (any_bad || q_bad) {
         // A key or value of the range, or a query of this wave, that the parts do
         // not serve: the rows over again in f32, straight from memory.
         clear();
 #pragma unroll 1
         for (uint32_t k0 = begin * kKeys + 16 * team; k0 < end * kKeys && k0 <= wave_last;
-             k0 += 16 * kTeams) {
+             k0 += 16 * TEAMS) {
             // 16 keys: scores of key 4q + r, operand key j.
             v4f s = {0, 0, 0, 0};
             const float *const kp = keys + size_t(min(k0 + j, k_end - 1)) * kv_width + 4 * q;
@@ -451,29 +456,31 @@ __global__ __launch_bounds__(kTeams * kThreads, 4) void gqa_flash_split_kernel(
             }
         }
     }
-    // The second team hands its rows to the first.
-    static_assert(kThreads * (4 * 16 + 2 * 4) <= sizeof(lds), "the teams' exchange");
-    v4f *const o_lds = reinterpret_cast<v4f *>(lds[0]) + tid;
-    float *const ml_lds = reinterpret_cast<float *>(lds[0] + 4 * 16 * kThreads) + tid;
-    if (team != 0) {
+    if constexpr (TEAMS == 2) {
+        // The second team hands its rows to the first.
+        static_assert(kThreads * (4 * 16 + 2 * 4) <= sizeof(lds), "the teams' exchange");
+        v4f *const o_lds = reinterpret_cast<v4f *>(lds[0]) + tid;
+        float *const ml_lds = reinterpret_cast<float *>(lds[0] + 4 * 16 * kThreads) + tid;
+        if (team != 0) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                o_lds[u * kThreads] = o[u];
+            ml_lds[0] = m;
+            ml_lds[kThreads] = l;
+        }
+        __syncthreads();
+        if (team != 0)
+            return;
+        const float m_other = ml_lds[0], m_new = fmaxf(m, m_other);
+        const float m_ref = m_new == -__builtin_inff() ? 0.0f : m_new;
+        const float w = __builtin_amdgcn_exp2f(m - m_ref);
+        const float w_other = __builtin_amdgcn_exp2f(m_other - m_ref);
+        m = m_new;
+        l = l * w + ml_lds[kThreads] * w_other;
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-            o_lds[u * kThreads] = o[u];
-        ml_lds[0] = m;
-        ml_lds[kThreads] = l;
+            o[u] = o[u] * w + o_lds[u * kThreads] * w_other;
     }
-    __syncthreads();
-    if (team != 0)
-        return;
-    const float m_other = ml_lds[0], m_new = fmaxf(m, m_other);
-    const float m_ref = m_new == -__builtin_inff() ? 0.0f : m_new;
-    const float w = __builtin_amdgcn_exp2f(m - m_ref);
-    const float w_other = __builtin_amdgcn_exp2f(m_other - m_ref);
-    m = m_new;
-    l = l * w + ml_lds[kThreads] * w_other;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-        o[u] = o[u] * w + o_lds[u * kThreads] * w_other;
     l = quad_sum(l);  // each lane holds its own keys' share
     if (!valid)
         return;
@@ -534,6 +541,11 @@ struct Grid {
     uint32_t tile_tokens, token_tiles, ranges, range_tiles;
 };
 
+// Key tiles per block up to which one team, without the exchange, is faster (us, two
+// teams and one: 40 tokens of 32 / 8 heads 10.6, 9.2, 128 tokens 12.7, 12.2; at four
+// tiles 200 tokens of 16 / 8 16.2, 16.8).
+constexpr uint32_t kOneTeam = 2;
+
 // Blocks the CUs hold at once: one each.
 constexpr uint32_t kResident = 256;
 
@@ -582,9 +594,15 @@ void launch_gqa_flash_split(hipStream_t stream, float *out, const float *query,
                             float *records)
 {
     const Grid d = grid_of(g, records != nullptr);
-    gqa_flash_split_kernel<<<d.token_tiles * d.ranges * g.key_value_heads, kTeams * kThreads, 0,
-                             stream>>>(out, query, key_cache, value_cache, g, d.tile_tokens,
-                                       d.token_tiles, d.ranges, d.range_tiles, records);
+    const uint32_t blocks = d.token_tiles * d.ranges * g.key_value_heads;
+    if (d.range_tiles <= kOneTeam)
+        gqa_flash_split_kernel<1><<<blocks, kThreads, 0, stream>>>(
+            out, query, key_cache, value_cache, g, d.tile_tokens, d.token_tiles, d.ranges,
+            d.range_tiles, records);
+    else
+        gqa_flash_split_kernel<2><<<blocks, 2 * kThreads, 0, stream>>>(
+            out, query, key_cache, value_cache, g, d.tile_tokens, d.token_tiles, d.ranges,
+            d.range_tiles, records);
     if (d.ranges > 1) {
         const uint32_t pairs = uint32_t(g.tokens) * g.query_heads;
         gqa_flash_merge_kernel<<<(pairs + 3) / 4, 256, 0, stream>>>(out, records, d.ranges, pairs);
